@@ -19,7 +19,7 @@
 // Logits kernel: workgroup = (token, run of keys); 4 wavefronts, each takes
 // a run of 16-key groups.  Per group: the 16 keys' 128 bytes (one contiguous
 // 2 KB block when the keys share a page) and scales, then per head tile one
-// v_mfma_scale_f32_16x16x128_f8f6f4 (unit scales) with A = q (16 heads x
+// v_mfma_f32_16x16x128_f8f6f4 with A = q (16 heads x
 // 128 dims), B = k^T (128 dims x 16 keys).  Lane (g, c) of D holds key c for
 // heads 4g + [0, 4) of each head tile, so the relu-weighted head sum is 4
 // clamps and 4 FMAs per tile and two cross-row swaps, the key's scale one
@@ -51,6 +51,9 @@ constexpr int kHeadDim = 128;
 constexpr int kMaxHeads = 64;
 constexpr int kLogitWaves = 4;
 constexpr int kLogitThreads = 64 * kLogitWaves;
+
+// Workgroup barrier for LDS traffic only (loads in flight stay in flight).
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 typedef float f32x4v __attribute__((ext_vector_type(4)));
 
@@ -105,13 +108,15 @@ __device__ __forceinline__ i32x8 key_operand(uint64_t k0, uint64_t k1, uint64_t 
 }
 
 // q . k for 16 heads x 16 keys over all 128 dims in one
-// v_mfma_scale_f32_16x16x128_f8f6f4 (both operands FP8 E4M3, unit E8M0
-// scales): lane (g, c) gives the same 32 dims of its head (A) and of its key
+// v_mfma_f32_16x16x128_f8f6f4 (both operands FP8 E4M3; zero scale operands
+// select the instruction without block scales): lane (g, c) gives the same 32 dims of its head (A) and of its key
 // (B), so every q byte meets the k byte of the same dim.
-__device__ __forceinline__ f32x4v dot128_fp8(const uint64_t (&q)[4], const i32x8& kb) {
-  const i32x8 qa = key_operand(q[0], q[1], q[2], q[3]);
+__device__ __forceinline__ f32x4v dot128_fp8(const i32x8& qa, const i32x8& kb) {
   const f32x4v zero = {0.f, 0.f, 0.f, 0.f};
-  return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(qa, kb, zero, 0, 0, 0, 127, 0, 127);
+  return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(qa, kb, zero, 0, 0, 0, 0, 0, 0);
+}
+__device__ __forceinline__ f32x4v dot128_fp8(const uint64_t (&q)[4], const i32x8& kb) {
+  return dot128_fp8(key_operand(q[0], q[1], q[2], q[3]), kb);
 }
 
 // The key's scale taken out of the head sum: relu(s d) = |s| relu(d') with
@@ -268,45 +273,113 @@ __global__ __launch_bounds__(kLogitThreads) void fp8_paged_mqa_logits_kernel(
 }
 
 // Rows that share one block table (the query rows of one request's prefill
-// chunk, each with its own causal length): workgroup = (run of kN 16-key
-// groups, 16 rows); wave w scores rows 4w .. 4w + 3 of the block over the
-// run, so each key group is loaded once per wave and used for 4 rows x
-// kTiles head tiles, and the four waves load the same groups (the later
-// waves' loads hit the CU's L1) -- the keys are read from L2 once per 16 rows
-// instead of once per row.  Same arithmetic per (row, key) as the per-token
-// kernel above; block sizes that are a multiple of 16 only.
-template <int kTiles, int kN>
-__global__ __launch_bounds__(kLogitThreads) void fp8_mqa_logits_rows_kernel(const LogitsArgs a, int num_tokens) {
+// chunk, each with its own causal length): workgroup = (run of up to kRowsRun
+// keys, 16 rows); wave w scores rows 4w .. 4w + 3.  Keys and scales go to
+// LDS in double-buffered chunks of 64 keys (wave w loads the chunk's group w
+// with whole-KB instructions, a chunk ahead), and every wave reads its B
+// operands there: one L1 access per 64 bytes of key and workgroup, where
+// operands loaded straight from memory cost one per 16-byte lane and wave.
+// Same arithmetic per (row, key) as the per-token kernel above, bit for bit;
+// block sizes that are a multiple of 16 only.
+//
+// Bound: issue.  A group of 16 keys costs a wave 8 products (4 rows x 2 head
+// tiles at 32 heads) and 64 clamps and FMAs; a loop of just these takes 155 ns
+// per group at three waves per SIMD (117 ns for the products, 75-90 for the
+// VALU work: a product holds the VALU for about half of its 32 cycles), and
+// this kernel 220 ns.  So: products without the scale operands (an unscaled
+// product holds the VALU for a third less time), issued two steps ahead of
+// their clamps with no wait between, operands read from LDS a group ahead,
+// masks and stores once per chunk (16 bytes per lane).  2048 rows x 65536
+// pools, 32 heads: 650 -> 465 us (2.35 PFLOP/s of FP8); with the top-512
+// 863 -> 706 us, 500 rows x 16000 pools 80.0 -> 65.6 us.
+constexpr int kRowsRun = 1024;         // keys of a workgroup: 64 groups, one per lane of the table lookup
+constexpr int kRowsChunk = 4;          // 16-key groups per chunk, one staged by each wave
+constexpr int kRowsBufs = 2;
+
+struct __attribute__((aligned(16))) RowsShared {
+  uint4 key[kRowsBufs][kRowsChunk][16 * 8];   // [group][key 8 + slot]: slot p ^ rows_swz(key) holds piece p
+  float sc[kRowsBufs][kRowsChunk][16];
+  float res[kLogitWaves][4][16 * kRowsChunk + 16];   // a wave's results by row (64 bytes apart in the banks)
+};
+
+__device__ __forceinline__ int rows_swz(int key) { return (key & 7) ^ ((key >> 3) & 1); }
+
+template <int kTiles>
+__global__ __launch_bounds__(kLogitThreads) __attribute__((amdgpu_waves_per_eu(kTiles == 1 ? 4 : kTiles == 2 ? 3 : 2)))
+void fp8_mqa_logits_rows_kernel(const LogitsArgs a, int num_tokens) {
   constexpr int kR = 4;        // rows per wave (row_sum4x4 leaves row g's sums in lane group g)
-  constexpr int kDepth = 4;
+  __shared__ RowsShared sh;
   const int lane = threadIdx.x & 63;
   const int w = uniform(threadIdx.x >> 6);
   const int g = lane >> 4, c = lane & 15;
   const int t0 = blockIdx.y * (kR * kLogitWaves) + kR * w;   // first row of this wave
   const int j_run = blockIdx.x * a.keys_per_wg;
-  const int j_end = j_run + 16 * kN < a.max_len ? j_run + 16 * kN : a.max_len;
-  const int n = (j_end - j_run + 15) / 16;
+  const int j_end = min(j_run + a.keys_per_wg, a.max_len);
   const int cap = a.max_blocks * a.block_size;
   int len[kR];
-  int len_max = 0;
 #pragma unroll
   for (int r = 0; r < kR; r++) {
-    int l = t0 + r < num_tokens ? a.ctx[t0 + r] : 0;
-    l = l < 0 ? 0 : l > cap ? cap : l;
-    len[r] = l;
-    len_max = len_max > l ? len_max : l;
+    const int l = t0 + r < num_tokens ? a.ctx[t0 + r] : 0;
+    len[r] = l < 0 ? 0 : l > cap ? cap : l;
   }
   const int my_len = g == 0 ? len[0] : g == 1 ? len[1] : g == 2 ? len[2] : len[3];   // row 4w + g
-
-  // page of each group's first key (lane i < n: group i; -1 past every row's context)
-  int blk_l = -1;
-  if (lane < n) {
-    const int j0 = j_run + 16 * lane;
-    if (j0 < len_max) blk_l = a.bt[j0 / a.block_size];
+  // the longest context of the workgroup's rows (the same in every wave)
+  int len_max = 0;
+  {
+    const int t = blockIdx.y * (kR * kLogitWaves) + c;
+    int l = t < num_tokens ? a.ctx[t] : 0;
+    l = l < 0 ? 0 : l > cap ? cap : l;
+    len_max = static_cast<int>(wave_max_u32(static_cast<uint32_t>(l)));
   }
+  // past every row's context the run is only written when cleaning
+  const int j_live = min(j_end, len_max);
+  const int chunks = j_live > j_run ? (j_live - j_run + 63) / 64 : 0;
+
+  // page and offset of group `lane`'s first key (page -1 past the contexts)
+  int blk_l = -1, off_l = 0;
+  {
+    const int j0 = j_run + 16 * lane;
+    if (j0 < j_live) {
+      const int b = j0 / a.block_size;
+      blk_l = a.bt[b];
+      off_l = j0 - b * a.block_size;
+    }
+  }
+  const bool page_ok = blk_l >= 0 && blk_l < a.num_blocks;
+  const uint64_t live = __ballot(page_ok);
+  blk_l = page_ok ? blk_l : 0;   // page 0 stands in for a page outside the cache
+  off_l = page_ok ? off_l : 0;
+
+  // Chunk ch's group w through registers into LDS: 16 keys x 8 pieces of 16
+  // bytes (each load instruction one contiguous KB), piece p of a key in its
+  // slot p ^ rows_swz(key).  A key of negative scale has its E4M3 sign bits
+  // flipped here and the scales become their factors (signed_key, key_factor).
+  uint4 st0, st1;
+  float st_sc;
+  auto load_group_w = [&](int ch) {
+    const int i = min(kRowsChunk * ch + w, 63);
+    const int blk = __builtin_amdgcn_readlane(blk_l, i);
+    const int off = __builtin_amdgcn_readlane(off_l, i);
+    const uint8_t* page = a.kv + static_cast<int64_t>(blk) * a.page_bytes;
+    const uint4* keys = reinterpret_cast<const uint4*>(page + static_cast<int64_t>(off) * kHeadDim);
+    st0 = keys[lane];
+    st1 = keys[64 + lane];
+    st_sc = reinterpret_cast<const float*>(page + static_cast<int64_t>(a.block_size) * kHeadDim)[off + c];
+  };
+  const int st_slot0 = 8 * (lane >> 3) + ((lane & 7) ^ rows_swz(lane >> 3));
+  const int st_slot1 = 64 + 8 * (lane >> 3) + ((lane & 7) ^ rows_swz(8 + (lane >> 3)));
+  auto write_group_w = [&](int ch) {
+    const int buf = ch % kRowsBufs;
+    const int neg = st_sc < 0.f ? static_cast<int>(0x80808080u) : 0;
+    const uint32_t f0 = __builtin_amdgcn_ds_bpermute(4 * (lane >> 3), neg);
+    const uint32_t f1 = __builtin_amdgcn_ds_bpermute(4 * (lane >> 3) + 32, neg);
+    sh.key[buf][w][st_slot0] = make_uint4(st0.x ^ f0, st0.y ^ f0, st0.z ^ f0, st0.w ^ f0);
+    sh.key[buf][w][st_slot1] = make_uint4(st1.x ^ f1, st1.y ^ f1, st1.z ^ f1, st1.w ^ f1);
+    if (lane < 16) sh.sc[buf][w][lane] = key_factor(st_sc);
+  };
 
   // q fragments (A operand) and weights of this lane's heads, per row
-  uint64_t qf[kR][kTiles][4];
+  i32x8 qf[kR][kTiles];
   float wv[kR][kTiles][4];
 #pragma unroll
   for (int r = 0; r < kR; r++) {
@@ -315,69 +388,100 @@ __global__ __launch_bounds__(kLogitThreads) void fp8_mqa_logits_rows_kernel(cons
     for (int ht = 0; ht < kTiles; ht++) {
       const uint4* qp = reinterpret_cast<const uint4*>(a.q + t * a.sq_t + (16 * ht + c) * a.sq_h + 16 * g);
       const uint4 lo = qp[0], hi = qp[4];
-      qf[r][ht][0] = (static_cast<uint64_t>(lo.y) << 32) | lo.x;
-      qf[r][ht][1] = (static_cast<uint64_t>(lo.w) << 32) | lo.z;
-      qf[r][ht][2] = (static_cast<uint64_t>(hi.y) << 32) | hi.x;
-      qf[r][ht][3] = (static_cast<uint64_t>(hi.w) << 32) | hi.z;
+      qf[r][ht] = i32x8{static_cast<int>(lo.x), static_cast<int>(lo.y), static_cast<int>(lo.z), static_cast<int>(lo.w),
+                        static_cast<int>(hi.x), static_cast<int>(hi.y), static_cast<int>(hi.z), static_cast<int>(hi.w)};
 #pragma unroll
       for (int i = 0; i < 4; i++) wv[r][ht][i] = a.w[t * a.sw_t + 16 * ht + 4 * g + i];
     }
   }
 
-  __shared__ float res[kLogitWaves][kR][16 * kN];
-  Group ring[kDepth];
-  // group i of the run, or past the run's end its last group again (loaded, not used)
-  auto load = [&](int i, Group& gr) {
-    const int ic = i < n ? i : n - 1;
-    load_group<true>(a, 0, j_run + 16 * ic, __builtin_amdgcn_readlane(blk_l, ic), len_max, g, c, gr);
+  // The wave's results of chunk ch, from sh.res to the logits: lane (g, c)
+  // stores keys 4c .. 4c + 3 of row 4w + g, as one 16-byte store where the
+  // rows are aligned and all four are written (inside the row's context, or
+  // anywhere in the run when cleaning).
+  const int limit = t0 + g < num_tokens ? (a.clean ? j_end : min(j_end, my_len)) : 0;
+  float* const out = a.logits + static_cast<int64_t>(min(t0 + g, num_tokens - 1)) * a.sl_t + j_run + 4 * c;
+  const bool vec = (reinterpret_cast<uintptr_t>(a.logits) & 15) == 0 && (a.sl_t & 3) == 0;   // runs start at multiples of 64
+  auto store_chunk = [&](int ch) {
+    const int j = j_run + 64 * ch + 4 * c;
+    float4 v = *reinterpret_cast<const float4*>(&sh.res[w][g][4 * c]);
+    float* const o = out + 64 * ch;
+    // a page outside the cache, or past the row's context: -inf
+    const int n = (live >> (kRowsChunk * ch + (c >> 2))) & 1 ? my_len - j : 0;
+    const float ninf = -__builtin_inff();
+    v.x = n > 0 ? v.x : ninf;
+    v.y = n > 1 ? v.y : ninf;
+    v.z = n > 2 ? v.z : ninf;
+    v.w = n > 3 ? v.w : ninf;
+    if (vec && j + 3 < limit) {
+      *reinterpret_cast<float4*>(o) = v;
+    } else {
+      if (j < limit) o[0] = v.x;
+      if (j + 1 < limit) o[1] = v.y;
+      if (j + 2 < limit) o[2] = v.z;
+      if (j + 3 < limit) o[3] = v.w;
+    }
   };
-  if (n > 0) {
+
+  if (chunks > 0) {
+    load_group_w(0);
+    write_group_w(0);
+    load_group_w(1);
+  }
+#pragma clang loop unroll(disable)
+  for (int ch = 0; ch < chunks; ch++) {
+    lds_barrier();   // chunk ch is in LDS, and every wave is done with chunk ch - 1's buffer
+    // the next chunk's write first: behind the stores its wait would include them
+    write_group_w(ch + 1);
+    if (ch > 0) store_chunk(ch - 1);
+    load_group_w(ch + 2);
+    // 4 groups x kR rows x kTiles products as one sequence: product m is
+    // issued kAhead steps before its clamps and FMAs, across the groups'
+    // boundaries too, so no step waits for a matrix result, and a group's
+    // operands leave LDS one group ahead.
+    const int buf = ch % kRowsBufs;
+    constexpr int kProducts = kR * kTiles;      // per group
+    constexpr int kAhead = 2;
+    i32x8 kb[2];
+    float sc[2];
+    auto read_group = [&](int i) {
+      const uint4* kp = &sh.key[buf][i][8 * c];
+      const uint4 lo = kp[g ^ rows_swz(c)], hi = kp[(4 + g) ^ rows_swz(c)];
+      kb[i & 1] = i32x8{static_cast<int>(lo.x), static_cast<int>(lo.y), static_cast<int>(lo.z), static_cast<int>(lo.w),
+                        static_cast<int>(hi.x), static_cast<int>(hi.y), static_cast<int>(hi.z), static_cast<int>(hi.w)};
+      sc[i & 1] = sh.sc[buf][i][c];
+    };
+    read_group(0);
+    f32x4v d[kAhead + 1];
+    float v[kR] = {};
 #pragma unroll
-    for (int s = 0; s < kDepth - 1; s++)
-      if (s < kN) load(s, ring[s]);
-#pragma unroll
-    for (int i = 0; i < kN; i++) {
-      if (i + kDepth - 1 < kN) load(i + kDepth - 1, ring[(i + kDepth - 1) % kDepth]);
-      if (i >= n) continue;   // uniform (the tail of the rows)
-      const Group& gr = ring[i % kDepth];
-      const int j = j_run + 16 * i + c;
-      float tot = 0.f;   // lane (g, c): row 4w + g at key j
-      if (gr.live) {
-        const uint64_t k0 = (static_cast<uint64_t>(gr.kd[0].y) << 32) | gr.kd[0].x;
-        const uint64_t k1 = (static_cast<uint64_t>(gr.kd[0].w) << 32) | gr.kd[0].z;
-        const uint64_t k2 = (static_cast<uint64_t>(gr.kd[1].y) << 32) | gr.kd[1].x;
-        const uint64_t k3 = (static_cast<uint64_t>(gr.kd[1].w) << 32) | gr.kd[1].z;
-        const i32x8 kb = signed_key(key_operand(k0, k1, k2, k3), gr.sc);
-        float v[kR] = {};
-#pragma unroll
-        for (int r = 0; r < kR; r++) {
-#pragma unroll
-          for (int ht = 0; ht < kTiles; ht++) {
-            const f32x4v d = dot128_fp8(qf[r][ht], kb);
-#pragma unroll
-            for (int e = 0; e < 4; e++) v[r] = __builtin_fmaf(wv[r][ht][e], relu_dot(d[e]), v[r]);
-          }
-        }
-        tot = key_factor(gr.sc) * row_sum4x4(v);
+    for (int m = 0; m < kRowsChunk * kProducts + kAhead; m++) {
+      if (m < kRowsChunk * kProducts) {
+        const int i = m / kProducts, q = m % kProducts;
+        d[m % (kAhead + 1)] = dot128_fp8(qf[q / kTiles][q % kTiles], kb[i & 1]);
+        if (q == kAhead && i + 1 < kRowsChunk) read_group(i + 1);   // the group before i is finished: its slot is free
       }
-      // page outside the cache, or past the row's context: -inf (written past
-      // the context only when cleaning, which the stores below decide)
-      res[w][g][16 * i + c] = gr.kok && j < my_len ? tot : -__builtin_inff();
+      if (m >= kAhead) {
+        const int i = (m - kAhead) / kProducts, q = (m - kAhead) % kProducts, r = q / kTiles, ht = q % kTiles;
+        const f32x4v dq = d[(m - kAhead) % (kAhead + 1)];
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[r] = __builtin_fmaf(wv[r][ht][e], relu_dot(dq[e]), v[r]);
+        if (q == kProducts - 1) {
+          sh.res[w][g][16 * i + c] = sc[i & 1] * row_sum4x4(v);   // lane (g, c): row 4w + g at key c
+#pragma unroll
+          for (int rr = 0; rr < kR; rr++) v[rr] = 0.f;
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
     }
   }
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  if (chunks > 0) store_chunk(chunks - 1);
+  if (a.clean) {   // the run past every row's context
 #pragma unroll
-  for (int r = 0; r < kR; r++) {
-    if (t0 + r >= num_tokens) break;   // uniform
-    float* out = a.logits + (t0 + r) * a.sl_t;
-#pragma unroll
-    for (int q = 0; q < (16 * kN + 63) / 64; q++) {
-      const int idx = 64 * q + lane;
-      const int j = j_run + idx;   // written inside the run, and past the row's context only when cleaning
-      if (idx < 16 * n && j < j_end && (j < len[r] || a.clean)) out[j] = res[w][r][idx];
-    }
+    for (int r = 0; r < kR; r++)
+      if (t0 + r < num_tokens)
+        for (int j = j_run + 64 * chunks + lane; j < j_end; j += 64)
+          a.logits[(t0 + r) * a.sl_t + j] = -__builtin_inff();
   }
 }
 
@@ -896,20 +1000,23 @@ extern "C" int glm53_fp8_paged_mqa_logits(const void* q, int64_t sq_t, int64_t s
   // group when groups straddle pages (block_size % 16 != 0).
   const bool al = block_size % 16 == 0;
   if (bt_stride == 0 && al && num_tokens >= 16) {
-    // one table shared by every row (a request's prefill chunk): 16 rows x 512 keys per workgroup
-    constexpr int kRowsN = 32;
+    // one table shared by every row (a request's prefill chunk): 16 rows x
+    // kRowsRun keys per workgroup, shorter runs while they leave fewer than
+    // 1024 workgroups (four per CU; a workgroup loads its 16 rows' queries
+    // once per run)
     LogitsArgs a{static_cast<const uint8_t*>(q), sq_t, sq_h, static_cast<const uint8_t*>(kv_cache), page_bytes,
                  static_cast<int>(block_size), static_cast<int>(num_blocks), weights, sw_t, context_lens,
                  block_table, 0, static_cast<int>(max_blocks), static_cast<int>(num_heads),
-                 static_cast<int>(max_len), 16 * kRowsN, logits, sl_t, clean_logits ? 1 : 0};
-    const dim3 grid(static_cast<unsigned>((max_len + 16 * kRowsN - 1) / (16 * kRowsN)),
-                    static_cast<unsigned>((num_tokens + 4 * kLogitWaves - 1) / (4 * kLogitWaves)));
+                 static_cast<int>(max_len), kRowsRun, logits, sl_t, clean_logits ? 1 : 0};
+    const int64_t row_blocks = (num_tokens + 4 * kLogitWaves - 1) / (4 * kLogitWaves);
+    while (a.keys_per_wg > 128 && row_blocks * ((max_len + a.keys_per_wg - 1) / a.keys_per_wg) < 1024) a.keys_per_wg /= 2;
+    const dim3 grid(static_cast<unsigned>((max_len + a.keys_per_wg - 1) / a.keys_per_wg), static_cast<unsigned>(row_blocks));
     void (*kernel)(LogitsArgs, int);
     switch (num_heads / 16) {
-      case 1: kernel = fp8_mqa_logits_rows_kernel<1, kRowsN>; break;
-      case 2: kernel = fp8_mqa_logits_rows_kernel<2, kRowsN>; break;
-      case 3: kernel = fp8_mqa_logits_rows_kernel<3, kRowsN>; break;
-      default: kernel = fp8_mqa_logits_rows_kernel<4, kRowsN>; break;
+      case 1: kernel = fp8_mqa_logits_rows_kernel<1>; break;
+      case 2: kernel = fp8_mqa_logits_rows_kernel<2>; break;
+      case 3: kernel = fp8_mqa_logits_rows_kernel<3>; break;
+      default: kernel = fp8_mqa_logits_rows_kernel<4>; break;
     }
     (void)hipGetLastError();
     hipLaunchKernelGGL(kernel, grid, dim3(kLogitThreads), 0, static_cast<hipStream_t>(stream), a,

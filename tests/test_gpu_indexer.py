@@ -425,3 +425,38 @@ def test_shared_table_rows_kernel(cuda, oracle, heads):
             n = torch.arange(pools, device=cuda)[None, :] < lens.clamp(max=pools)[:, None].long()
             assert torch.equal(got[n], ref[n])
         check_logits(oracle, got, q, cache, w, lens, shared.contiguous(), pools, clean, rows=range(0, T, 6))
+
+
+@pytest.mark.parametrize("heads,bs,pools,T", [(16, 16, 1023, 16), (48, 48, 1025, 33), (32, 64, 64, 17),
+                                              (64, 128, 2049, 64), (32, 16, 15, 20)])
+def test_shared_table_run_edges(cuda, heads, bs, pools, T):
+    """The row-tiled kernel at its runs' and chunks' edges (1024 and 64 keys):
+    row counts around its 16-row blocks, odd row lengths (logits rows not
+    16-byte aligned, scalar stores), pages of one group and of three, a NaN
+    and a negative scale, a page outside the cache -- bit-identical to the
+    per-token kernel, and positions past a row's context left as they were
+    when not cleaning."""
+    import torch
+    from sparse_indexer import fp8_paged_mqa_logits
+    g = torch.Generator(device=cuda).manual_seed(7000 + pools)
+    per_req = (pools + bs - 1) // bs
+    cache, nb = W.indexer_cache(cuda, g, (per_req + 2) * bs, bs, page_pad=16)
+    pages = torch.as_strided(cache, (nb, cache.stride(0)), (cache.stride(0), 1))
+    sc = pages[:, bs * 128: bs * 132].contiguous().view(torch.float32)
+    sc[0, 0], sc[nb - 1, 1], sc[1, 2] = float("nan"), -sc[nb - 1, 1], 0.0
+    pages[:, bs * 128: bs * 132] = sc.view(torch.uint8)
+    table = torch.randperm(nb, generator=g, device=cuda).to(torch.int32)[:per_req]
+    if per_req > 2:
+        table[1] = nb
+    lens = torch.randint(0, pools + 1, (T,), generator=g, device=cuda, dtype=torch.int32)
+    lens[0], lens[T - 1] = pools + 9, 0
+    q = (torch.randn(T, 1, heads, 128, generator=g, device=cuda) * 60).to(torch.float8_e4m3fn)
+    w = (torch.randn(T, heads, generator=g, device=cuda) * heads ** -0.5).contiguous()
+    shared = table[None, :].expand(T, per_req)
+    log_case("indexer shared-table edges", heads, bs, pools, T)
+    for clean in (True, False):
+        got = fp8_paged_mqa_logits(q, cache, w, lens, shared, pools, clean_logits=clean)
+        ref = fp8_paged_mqa_logits(q, cache, w, lens, shared.contiguous(), pools, clean_logits=clean)
+        for r in range(T):
+            n = pools if clean else min(int(lens[r]), per_req * bs, pools)
+            assert torch.equal(got[r, :n], ref[r, :n]), f"row {r}"
