@@ -492,7 +492,6 @@ constexpr int kChunkThreadsWide = 1024;   // chunk workgroups of the few-rows pl
 constexpr int kFinalThreads = 1024;
 constexpr int kSweepThreads = 1024;
 constexpr int kSweepKeys = 32;                      // keys per thread per sweep
-constexpr int kSweep = kSweepThreads * kSweepKeys;  // positions per sweep (32768)
 
 struct TopkArgs {
   const float* logits;      // [rows][*], row stride sl
@@ -602,7 +601,7 @@ struct Threshold {
 // for_keys(f) calls f(key) for every key of this thread; the keys matching
 // the shared bits must number at least k.  The caller has zeroed both
 // histograms (clear_hist) before the call.
-template <int kThreads, class ForKeys>
+template <int kThreads, int kMaxPasses = 3, class ForKeys>
 __device__ Threshold radix_threshold(SelShared<kThreads>& sh, ForKeys for_keys, uint32_t k, uint32_t kmin,
                                      uint32_t kmax) {
   constexpr int kWaves = kThreads / 64;
@@ -618,7 +617,7 @@ __device__ Threshold radix_threshold(SelShared<kThreads>& sh, ForKeys for_keys, 
   int top = 32 - __clz(static_cast<int>(diff));   // bits [top, 32) are shared
   uint32_t pmask = top == 32 ? 0u : ~((1u << top) - 1u);
   uint32_t prefix = kmax & pmask, need = k;
-  for (int pass = 0; top > 0; pass++) {
+  for (int pass = 0; top > 0 && pass < kMaxPasses; pass++) {
     const int width = top < 12 ? top : 12;
     const int shift = top - width;
     top = shift;
@@ -893,41 +892,306 @@ __global__ __launch_bounds__(kFinalThreads) void topk_final_kernel(
   }, &n_eq, &n_sel);
 }
 
-// Rows too long for the two stages: one workgroup per row re-reads the row
-// (from L2) in sweeps of 32768 positions for each radix pass and for the
+// The k largest of one row of len > k positions by re-reading it (from L2)
+// in sweeps of kThreads * P positions, for each radix pass and for the
 // compaction, which carries its counts from sweep to sweep.
-__global__ __launch_bounds__(kSweepThreads) void topk_sweep_kernel(const TopkArgs a) {
-  __shared__ SelShared<kSweepThreads> sh;
-  const int row = blockIdx.x, tid = threadIdx.x;
-  const int len = clamp_len(a, row);
-  const int k = a.k;
-  int32_t* out = a.out + row * a.so;
-  if (len <= k) {
-    for (int i = tid; i < k; i += kSweepThreads) out[i] = i < len ? i : -1;
-    return;
-  }
-  const float* x = a.logits + row * a.sl;
+template <int kThreads, int P>
+__device__ void sweep_row(SelShared<kThreads>& sh, const float* x, int len, int k, bool vec, int32_t* out) {
+  constexpr int kSweep = kThreads * P;
+  const int tid = threadIdx.x;
   const int sweeps = (len + kSweep - 1) / kSweep;
   clear_hist(sh);
   const Threshold t = radix_threshold(sh, [&](auto f) {
     for (int sw = 0; sw < sweeps; sw++) {
-      uint32_t kk[kSweepKeys];
-      load_row_keys<kSweepKeys>(x + sw * kSweep, len - sw * kSweep, tid * kSweepKeys, a.vec, kk);
+      uint32_t kk[P];
+      load_row_keys<P>(x + sw * kSweep, len - sw * kSweep, tid * P, vec, kk);
       for_each_key(kk, f);
     }
   }, static_cast<uint32_t>(k), 0u, ~0u);
   uint32_t eq_seen = 0, written = 0;
   for (int sw = 0; sw < sweeps; sw++) {
-    uint32_t kk[kSweepKeys];
+    uint32_t kk[P];
     const int base = sw * kSweep;
-    load_row_keys<kSweepKeys>(x + base, len - base, tid * kSweepKeys, a.vec, kk);
+    load_row_keys<P>(x + base, len - base, tid * P, vec, kk);
     uint32_t n_eq, n_sel;
     emit_selected(sh, kk, t, eq_seen, written, [&](uint32_t o, int j) {
-      if (o < static_cast<uint32_t>(k)) out[o] = base + tid * kSweepKeys + j;
+      if (o < static_cast<uint32_t>(k)) out[o] = base + tid * P + j;
     }, &n_eq, &n_sel);
     eq_seen += n_eq;
     written += n_sel;
     __syncthreads();   // the next sweep's scan rewrites sh.wsum
+  }
+}
+
+// Rows too long for the two stages: one workgroup per row, in sweeps.
+__global__ __launch_bounds__(kSweepThreads) void topk_sweep_kernel(const TopkArgs a) {
+  __shared__ SelShared<kSweepThreads> sh;
+  const int row = blockIdx.x;
+  const int len = clamp_len(a, row);
+  const int k = a.k;
+  int32_t* out = a.out + row * a.so;
+  if (len <= k) {
+    for (int i = threadIdx.x; i < k; i += kSweepThreads) out[i] = i < len ? i : -1;
+    return;
+  }
+  sweep_row<kSweepThreads, kSweepKeys>(sh, a.logits + row * a.sl, len, k, a.vec, out);
+}
+
+// One workgroup per row that looks at each key once.  A sample of 4096 keys
+// gives a bound T below the k-th largest key (the sample's rank k * 4096 /
+// len plus eight times its square root, so that 1.3 k to 2.5 k of the row's keys
+// lie at or above T); one pass over the row appends their positions to a list
+// in LDS; the radix select runs on the list alone; bitmaps of the row put the
+// selection in position order.  A pass over the row costs about 6 VALU
+// instructions per key, where the radix passes and the compaction of the
+// chunk stage cost 25, and nothing but the selection is written: 2048 rows x
+// 65536 positions read their 537 MB in 150 us (chunk and final stages 251).
+// When the bound's bin holds more than the list (heavy ties), the sample's exact
+// key of that rank takes its place, and if the keys above it are too few the
+// first positions equal to it complete them; a sample that still misleads
+// sends the row through sweep_row.  So ties cost a second pass (64 rows x 65536
+// of three distinct values 31 -> 29 us, 1 row 19 -> 28, one value everywhere 8
+// -> 22).
+constexpr int kListKeys = 4096;       // sample size and list capacity
+constexpr int kRowMaxLen = 131072;    // two bitmaps in the histograms' LDS
+constexpr int kRowMaxK = 1024;
+
+__device__ __forceinline__ float key_value(uint32_t key) {   // inverse of order_key (key 0: a NaN)
+  return __uint_as_float((key & 0x80000000u) ? key ^ 0x80000000u : ~key);
+}
+
+template <int kThreads>
+__global__ __launch_bounds__(kThreads) void topk_row_kernel(
+    const float* p_logits, int64_t p_sl, const int32_t* p_lengths, int p_max_len, int p_k, int p_vec,
+    int32_t* p_out, int64_t p_so) {
+  constexpr int P = kListKeys / kThreads;      // list keys per thread
+  constexpr int kRuns = P / 4;                 // sampled runs of 4 per thread
+  constexpr int kVecs = 4;                     // 4-key loads per thread and step of the pass over the row
+  __shared__ SelShared<kThreads> sh;
+  __shared__ int32_t list[kListKeys];
+  __shared__ uint32_t listed;
+  const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+  const int len = clamp_len(p_lengths, p_max_len, row);
+  const int k = p_k;
+  const float* x = p_logits + row * p_sl;
+  int32_t* out = p_out + row * p_so;
+  if (len <= k) {   // every valid position is selected (uniform)
+    for (int i = tid; i < k; i += kThreads) out[i] = i < len ? i : -1;
+    return;
+  }
+  uint32_t kk[P];
+  if (len <= kListKeys) {   // the whole row as one list, in position order
+    float f[P];
+    issue_row_loads<P>(x, len, tid * P, p_vec, f);
+    clear_hist(sh);
+    form_keys<P>(f, len, tid * P, kk);
+    uint32_t kmin = ~0u, kmax = 0u;
+#pragma unroll
+    for (int j = 0; j < P; j++)
+      if (tid * P + j < len) { kmin = min(kmin, kk[j]); kmax = max(kmax, kk[j]); }
+    const Threshold t = radix_threshold(sh, [&](auto f) { for_each_key(kk, f); }, static_cast<uint32_t>(k), kmin, kmax);
+    uint32_t n_eq, n_sel;
+    emit_selected(sh, kk, t, 0u, 0u, [&](uint32_t o, int j) {
+      if (o < static_cast<uint32_t>(k)) out[o] = tid * P + j;
+    }, &n_eq, &n_sel);
+    return;
+  }
+
+  // The pass over the row: positions of the keys that `takes` picks go to the
+  // list, and to `listed` their number (an unfinished one past the capacity).
+  constexpr int kStep = kThreads * 4 * kVecs;
+  auto load_step = [&](int base, float4 (&f)[kVecs]) {
+#pragma unroll
+    for (int q = 0; q < kVecs; q++) {
+      const int i = base + (q * kThreads + tid) * 4;
+      if (p_vec && i + 4 <= len) {
+        f[q] = *reinterpret_cast<const float4*>(x + i);
+      } else {
+        const float nan = __builtin_nanf("");
+        f[q].x = i < len ? x[i] : nan;
+        f[q].y = i + 1 < len ? x[i + 1] : nan;
+        f[q].z = i + 2 < len ? x[i + 2] : nan;
+        f[q].w = i + 3 < len ? x[i + 3] : nan;
+      }
+    }
+  };
+  auto hits_of = [&](const float4 (&f)[kVecs], auto takes) {
+    uint32_t hits = 0;
+#pragma unroll
+    for (int q = 0; q < kVecs; q++) {
+      hits |= takes(f[q].x) ? 1u << (4 * q) : 0u;
+      hits |= takes(f[q].y) ? 2u << (4 * q) : 0u;
+      hits |= takes(f[q].z) ? 4u << (4 * q) : 0u;
+      hits |= takes(f[q].w) ? 8u << (4 * q) : 0u;
+    }
+    return hits;
+  };
+  auto hit_pos = [&](int base, int b) { return base + ((b >> 2) * kThreads + tid) * 4 + (b & 3); };
+  auto list_keys = [&](auto takes) {
+    float4 cur[kVecs], nxt[kVecs];
+    load_step(0, cur);
+    bool room = true;   // uniform over the wave
+    for (int base = 0; base < len && room; base += kStep) {
+      if (base + kStep < len) load_step(base + kStep, nxt);
+      uint32_t hits = hits_of(cur, takes);
+      const uint32_t n = __popc(hits);
+      const uint32_t incl = wave_incl_scan(n);
+      const uint32_t total = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(incl), 63));
+      if (total) {   // uniform over the wave
+        uint32_t at = 0;
+        if (lane == 63) at = atomicAdd(&listed, total);
+        at = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(at), 63));
+        room = at <= kListKeys;   // else overflown: the count says so
+        at += incl - n;
+        while (hits) {
+          const int b = __builtin_ctz(hits);
+          hits &= hits - 1;
+          if (at < kListKeys) list[at] = hit_pos(base, b);
+          at++;
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < kVecs; q++) cur[q] = nxt[q];
+    }
+    __syncthreads();
+    return static_cast<int>(listed);
+  };
+
+  // ---- the bound T from a sample: runs of 4 keys at 1024 even places
+  auto load_sample = [&](float (&f)[P]) {
+#pragma unroll
+    for (int q = 0; q < kRuns; q++) {
+      const float* s = x + ((static_cast<uint32_t>(q * kThreads + tid) * static_cast<uint32_t>(len) / (kListKeys / 4)) & ~3u);
+      if (p_vec) {
+        const float4 v = *reinterpret_cast<const float4*>(s);
+        f[4 * q] = v.x; f[4 * q + 1] = v.y; f[4 * q + 2] = v.z; f[4 * q + 3] = v.w;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; e++) f[4 * q + e] = s[e];
+      }
+    }
+  };
+  auto sample_keys = [&](const float (&f)[P], uint32_t& kmin, uint32_t& kmax) {
+    kmin = ~0u;
+    kmax = 0u;
+#pragma unroll
+    for (int j = 0; j < P; j++) {
+      kk[j] = order_key(f[j]);
+      kmin = min(kmin, kk[j]);
+      kmax = max(kmax, kk[j]);
+    }
+  };
+  const float mean = static_cast<float>(k) * kListKeys / static_cast<float>(len);
+  const uint32_t rank = static_cast<uint32_t>(min(static_cast<int>(mean + 8.f * __builtin_sqrtf(mean) + 8.f), kListKeys));
+  uint32_t kmin, kmax;
+  float bound;
+  {
+    float f[P];
+    load_sample(f);
+    clear_hist(sh);
+    if (tid == 0) listed = 0;
+    sample_keys(f, kmin, kmax);
+    // one pass: the bin the rank falls in, whole
+    const Threshold t = radix_threshold<kThreads, 1>(sh, [&](auto f) { for_each_key(kk, f); }, rank, kmin, kmax);
+    bound = key_value(t.thr & t.pmask);
+  }
+  int n_list = list_keys([&](float v) { return v >= bound; });   // a NaN bound lists none
+  uint32_t ties = ~0u;   // the key whose first positions complete the list (none: the list holds the top k)
+  if (n_list > kListKeys) {   // uniform: many keys in the bin -- the sample's exact key of that rank, and the keys above it
+    float f[P];
+    load_sample(f);
+    clear_hist(sh);
+    sample_keys(f, kmin, kmax);
+    const Threshold t = radix_threshold(sh, [&](auto f) { for_each_key(kk, f); }, rank, kmin, kmax);
+    if (tid == 0) listed = 0;
+    __syncthreads();
+    n_list = list_keys([&](float v) { return order_key(v) > t.thr; });
+    if (n_list < k) ties = t.thr;
+  }
+  uint32_t* gt = sh.hist[0];   // later: a bitmap of the keys above the threshold and one of those at it
+  uint32_t* eq = sh.hist[1];
+  const int words = (len + 31) / 32;
+  if (ties != ~0u) {
+    // The list holds every key above `ties`: the first k - n_list positions
+    // of that key complete it, collected step by step from the row's start.
+    for (int i = tid; i < words; i += kThreads) gt[i] = eq[i] = 0u;
+    if (tid == 0) listed = 0;
+    __syncthreads();
+    for (int i = tid; i < n_list; i += kThreads) atomicOr(&gt[list[i] >> 5], 1u << (list[i] & 31));
+    int found = 0;
+    for (int base = 0; base < len && found < k - n_list; base += kStep) {
+      float4 cur[kVecs];
+      load_step(base, cur);
+      uint32_t hits = hits_of(cur, [&](float v) { return order_key(v) == ties; });
+      const uint32_t n = wave_incl_scan(__popc(hits));
+      if (lane == 63 && n) atomicAdd(&listed, n);
+      while (hits) {
+        const int b = __builtin_ctz(hits);
+        hits &= hits - 1;
+        const int p = hit_pos(base, b);
+        if (p < len) atomicOr(&eq[p >> 5], 1u << (p & 31));   // a NaN key (0) also stands past the row's end
+      }
+      __syncthreads();
+      found = static_cast<int>(listed);
+      __syncthreads();
+    }
+    if (found < k - n_list) ties = ~0u;   // uniform
+  }
+  if (ties == ~0u && (n_list < k || n_list > kListKeys)) {   // uniform: the sample misled
+    __syncthreads();
+    sweep_row<kThreads, P>(sh, x, len, k, p_vec, out);
+    return;
+  }
+  uint32_t need = static_cast<uint32_t>(k - n_list);   // of the keys at the threshold
+  if (ties == ~0u) {
+    // ---- the k largest of the list
+    int pos[P];
+#pragma unroll
+    for (int j = 0; j < P; j++) pos[j] = list[j * kThreads + tid < n_list ? j * kThreads + tid : 0];
+    float f[P];
+#pragma unroll
+    for (int j = 0; j < P; j++) f[j] = x[pos[j]];
+    clear_hist(sh);
+    kmin = ~0u;
+    kmax = 0u;
+#pragma unroll
+    for (int j = 0; j < P; j++) {
+      const bool ok = j * kThreads + tid < n_list;
+      kk[j] = ok ? order_key(f[j]) : 0u;
+      if (ok) { kmin = min(kmin, kk[j]); kmax = max(kmax, kk[j]); }
+    }
+    const Threshold t = radix_threshold(sh, [&](auto f) { for_each_key(kk, f); }, static_cast<uint32_t>(k), kmin, kmax);
+
+    need = t.need;
+    // the bitmaps take the histograms' place (their last reader is behind a barrier)
+    for (int i = tid; i < words; i += kThreads) gt[i] = eq[i] = 0u;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < P; j++) {
+      const uint32_t m = kk[j] & t.pmask;
+      if (kk[j] != 0u && m >= t.thr) atomicOr(m > t.thr ? &gt[pos[j] >> 5] : &eq[pos[j] >> 5], 1u << (pos[j] & 31));
+    }
+  }
+  __syncthreads();
+  // ---- the selection in position order
+  const int per = (words + kThreads - 1) / kThreads;   // consecutive words of this thread
+  const int w0 = min(tid * per, words), w1 = min(w0 + per, words);
+  uint32_t n = 0;
+  for (int i = w0; i < w1; i++) n += (static_cast<uint32_t>(__popc(gt[i])) << 16) | static_cast<uint32_t>(__popc(eq[i]));
+  uint32_t all;
+  const uint32_t before = block_excl_scan(sh, n, &all);
+  uint32_t r = before & 0xffffu;                       // keys at the threshold seen so far
+  uint32_t o = (before >> 16) + min(r, need);
+  for (int i = w0; i < w1; i++) {
+    const uint32_t g = gt[i], e = eq[i];
+    uint32_t bits = g | e;
+    while (bits) {
+      const int b = __builtin_ctz(bits);
+      bits &= bits - 1;
+      const bool at = (e >> b) & 1;
+      if (!at || r < need) out[o++] = 32 * i + b;
+      r += at;
+    }
   }
 }
 
@@ -1098,6 +1362,21 @@ TopkPlan plan_topk(int64_t num_rows, int64_t max_len, int64_t k) {
   return best;
 }
 
+// Rows that topk_row_kernel takes whatever plan_topk says of them (its
+// workspace is asked for all the same and stays unused).  Against the chunk
+// and final stages, k = 512: 2048 rows x 65536 positions 251 -> 150 us, x
+// 16384 87 -> 50, 500 x 16000 27 -> 16.3, 48 x 12000 17.8 -> 10.2, 16 x 65536
+// 19.4 -> 13.9, 1 x 16384 12.2 -> 10.0.  A few long rows keep the two stages: one
+// compute unit streams a row that other XCDs have just written more slowly than
+// several do (a one-token decode layer over 65536 pools 40.1 -> 42.3 us with
+// this kernel, 8 tokens over 32768 79.4 -> 79.7), whatever a repeated call alone
+// says (14.0 -> 12.5).  512 threads leave three rows to a CU where many short
+// rows queue (2048 x 8192: 35 us against 48 with 1024 threads, x 16384 50 / 53, x
+// 32768 98 / 95; below 256 rows each has a CU to itself and 1024 threads are ahead).
+bool row_plan(int64_t num_rows, int64_t max_len, int64_t k) {
+  return max_len > kListKeys && max_len <= kRowMaxLen && k <= kRowMaxK && (max_len <= 16384 || num_rows >= 16);
+}
+
 int64_t topk_ws_bytes(const TopkPlan& p, int64_t rows, int64_t k) {
   if (p.mode != TopkPlan::kChunked) return 0;
   return (rows * p.chunks * k * 8 + 255) / 256 * 256;
@@ -1149,6 +1428,12 @@ extern "C" int glm53_indexer_topk(const float* logits, int64_t sl, const int32_t
   const hipStream_t st = static_cast<hipStream_t>(stream);
   const dim3 rows_grid(static_cast<unsigned>(num_rows));
   (void)hipGetLastError();
+  if (row_plan(num_rows, max_len, k)) {
+    const bool narrow = num_rows >= 256 && max_len <= 24576;
+    hipLaunchKernelGGL((narrow ? topk_row_kernel<512> : topk_row_kernel<1024>), rows_grid, dim3(narrow ? 512 : 1024), 0,
+                       st, a.logits, a.sl, a.lengths, a.max_len, a.k, a.vec ? 1 : 0, a.out, a.so);
+    return static_cast<int>(hipGetLastError());
+  }
   if (plan.mode == TopkPlan::kSweepMode) {
     hipLaunchKernelGGL(topk_sweep_kernel, rows_grid, dim3(kSweepThreads), 0, st, a);
     return static_cast<int>(hipGetLastError());

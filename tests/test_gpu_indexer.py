@@ -460,3 +460,41 @@ def test_shared_table_run_edges(cuda, heads, bs, pools, T):
         for r in range(T):
             n = pools if clean else min(int(lens[r]), per_req * bs, pools)
             assert torch.equal(got[r, :n], ref[r, :n]), f"row {r}"
+
+
+@pytest.mark.parametrize("rows,n,k", [(9, 4097, 512), (9, 5001, 1024), (270, 8192, 512), (9, 12001, 1), (9, 65536, 1024),
+                                      (17, 131072, 512), (9, 131073, 512), (9, 20000, 1025)])
+def test_topk_filtered_rows(cuda, oracle, rows, n, k):
+    """The one-workgroup selection that filters a row by a sampled bound, at
+    the edges of its range (4097 and 131072 positions, k = 1024, unaligned
+    rows, rows shorter than its list or than k, 512 and 1024 threads) and the
+    plans just past them, on rows whose sample says little: few distinct
+    values, one value, NaN or -inf almost everywhere, ascending, a block of
+    large keys, both zeros."""
+    import torch
+    from sparse_indexer import indexer_topk
+    g = torch.Generator(device=cuda).manual_seed(n + k)
+    x = torch.randn(rows, n, generator=g, device=cuda)
+    x[1] = torch.randint(0, 3, (n,), generator=g, device=cuda).float()
+    x[2] = -1.5
+    x[3] = torch.where(torch.rand(n, generator=g, device=cuda) < 0.98, torch.full_like(x[3], float("nan")), x[3])
+    x[4] = torch.where(torch.rand(n, generator=g, device=cuda) < 0.9, torch.full_like(x[4], -float("inf")), x[4])
+    x[5] = torch.arange(n, device=cuda, dtype=torch.float32)
+    x[6, n // 3: n // 3 + k] += 50.0
+    x[7] = torch.where(torch.rand(n, generator=g, device=cuda) < 0.5, torch.zeros_like(x[7]), -torch.zeros_like(x[7]))
+    x[7, ::97] = 1.0
+    lens = torch.full((rows,), n, dtype=torch.int32, device=cuda)
+    lens[8:] = torch.randint(1, n + 1, (rows - 8,), generator=g, device=cuda, dtype=torch.int32)
+    lens[8] = k
+    log_case("indexer top-k filtered rows", rows, n, k)
+    got = indexer_topk(x, lens, k).cpu().numpy()
+    check = list(range(min(rows, 40)))
+    want = oracle.indexer_topk(x[check].cpu().numpy(), lens[check].cpu().numpy(), k)
+    assert np.array_equal(got[check], want)
+    if rows > 40:   # the rest against the library's own threshold: k-th largest value and everything above it
+        xs, ls = x[40:].cpu().numpy(), lens[40:].cpu().numpy()
+        for r in range(xs.shape[0]):
+            m = min(int(ls[r]), k)
+            sel = got[40 + r, :m]
+            assert (np.diff(sel) > 0).all() and sel[-1] < ls[r] and (got[40 + r, m:] == -1).all()
+            assert np.array_equal(np.sort(xs[r, sel]), np.sort(xs[r, :ls[r]])[-m:])
