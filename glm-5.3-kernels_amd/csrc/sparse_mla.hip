@@ -37,10 +37,10 @@
 //   * V^T comes from the same gathered rows: each wave stores its bf16 slice
 //     row-major in LDS and reads it back with ds_read_b64_tr_b16 (two reads
 //     per 16x32 operand).  O^T accumulates in 8 MFMA tiles per wave.
-//   * Splits longer than one chunk (the prefill-shaped call's single split
-//     of 2176 keys per token) run sparse_mla_pair_kernel instead: two waves
-//     per (token, 16-head group) share one online-softmax stream over the
-//     split's tiles in order.
+//   * Splits longer than one chunk (batches of more than about 30 tokens, the
+//     prefill-shaped call's single split of 2176 keys per token) run
+//     sparse_mla_rows_kernel instead: every wave of a workgroup takes 16 whole
+//     rows of a unit of 64 or 128 keys, then a slice of the output.
 //   * Workgroups are numbered so that a token's splits share an XCD (its L2
 //     holds the token's q and indices, and the merge kernel is numbered the
 //     same way); see sparse_mla_kernel.
@@ -661,12 +661,11 @@ __global__ __launch_bounds__(SplitShape<kG>::kThreads) void sparse_mla_kernel(
 }
 
 // ---------------------------------------------------------------- long splits: waves in pairs
-// Splits of more than one chunk of flat-row indices (the prefill-shaped call:
-// one split of 2176 keys per token) take this kernel.  One workgroup of two
-// waves per (split, token, 16-head group) runs a single online-softmax stream
-// over the split's 32-key tiles in order -- the loop structure of
-// _sparse_mla_compute_tile with BLOCK_N = 32 -- and the two waves split the
-// latent: wave w gathers, converts and multiplies latents [256 w, 256 w + 256)
+// Splits of more than one chunk where sparse_mla_rows_kernel does not take
+// them (rows_waves).  One workgroup of two waves per (split, token, 16-head
+// group) runs a single online-softmax stream over the split's 32-key tiles in
+// order -- the loop structure of _sparse_mla_compute_tile with BLOCK_N = 32 --
+// and the two waves split the latent: wave w gathers, converts and multiplies latents [256 w, 256 w + 256)
 // of every key.
 //   * S^T = K Q^T per 16-key half on v_mfma_f32_16x16x32_bf16 over the wave's
 //     256 latents (8 K-steps); the two waves' partial S^T meet in LDS (one
@@ -969,6 +968,311 @@ void sparse_mla_pair_kernel(const MlaArgs a) {
   }
 }
 
+// ---------------------------------------------------------------- long splits: 16 keys per wave
+// Splits of more than 256 keys.  One workgroup of kW waves (4 or 8) per
+// (split, token, 16-head group) walks the split in units of 16 kW keys with
+// one online softmax:
+//   * Wave w gathers keys 16 w .. 16 w + 15 of the unit whole: each load
+//     instruction takes two rows' 512 code bytes, 32 lanes to a row, so a row
+//     costs the L1 8 accesses of 64 bytes instead of 33 of 16.  It converts
+//     them to bf16 in LDS and multiplies q with its own 16 rows over all 512
+//     latents (16 K-steps): no partial scores are exchanged and no softmax is
+//     repeated in another wave.
+//   * P: every lane holds the scores of 4 keys for its head; each wave's
+//     bf16(p * scale) is half of a B operand of O^T = V^T P^T and goes through
+//     LDS to the others, computed against the running maximum of the units
+//     before, so that the common unit has one barrier between scores and
+//     products and no rescaling.  Where a unit raises a head's maximum
+//     (every wave sees the unit's maxima and takes the same branch) the
+//     accumulator is rescaled and the weights are computed again.  Letting
+//     the maximum lag by up to 2^2, 2^8 or 2^40 saved nothing and cost
+//     precision: the largest key's weight is exactly 1 only against its own
+//     score (2^40: twice the squared error where one key dominates).
+//   * PV: wave w computes latents (512 / kW) w + [0, 512 / kW) from all rows
+//     in LDS (ds_read_b64_tr_b16), then a barrier frees the rows.
+//   * Row gathers run one unit ahead, table lookups two, index loads three.
+// LDS rows are 1 KB; even 16-byte chunks fill a row's first half, odd ones the
+// second (so a row's write instruction is contiguous), and the place's low four
+// bits are XORed with a code of the row in which the 16 rows of an operand
+// read, the 8 rows x 2 chunks of a transposing read and the halves of either
+// pass differ: SQ_LDS_BANK_CONFLICT is 0 but for the maxima.
+//
+// Bound: a lone wave issues an instruction about every six cycles, and two per
+// SIMD about every 2.6 each, so up to 256 workgroups the kernel's 480
+// instructions per wave and unit set the time, with two barriers; from about
+// 1000 tokens on the row gathers do (T=1024: 164 us from L2-resident rows, 204
+// over a 262144-row cache, 5.8 TB/s of row bytes).  Against the pair kernel
+// below (262144-row cache, 2176 indices, us): 128 tokens 78 -> 40 (2 splits,
+// with the merge of few splits), 256 105 -> 57, 300 142 -> 89, 512 145 -> 107, 1100
+// 289 -> 248, 2048 418 -> 388; 48 tokens in 5 splits 36.2 -> 22.4.
+// 128-key units of 8 waves against 64-key units of 4, one split: 256 tokens 57
+// / 66, 300 100 / 89, 512 110 / 107, 640 154 / 158, 1024 214 / 204 -- by the rounds
+// they take on the compute units (one workgroup of 8 waves each, or two of 4).
+constexpr int kRowBf16Bytes = kLatent * 2;    // a converted row in LDS
+
+template <int kW>
+struct __attribute__((aligned(1024))) RowsShared {
+  uint16_t v[16 * kW][kLatent];     // the unit's rows in bf16 (rows_vofs)
+  uint2 p[kW][64];                  // each wave's part of the P^T operand
+  float mx[kHeads][kW];             // each wave's maximum per head (l at the end)
+};
+
+// Byte offset of the 16-byte chunk `chunk` (latents 8 chunk + [0, 8)) of row
+// `row`: even chunks fill the row's first half, odd chunks the second, and
+// the low four bits of the place are XORed with a code of the row and the half.
+__device__ __forceinline__ int rows_f(int row) {
+  return (row & 3) ^ (row & 4 ? 12 : 0) ^ (row & 8);
+}
+__device__ __forceinline__ int rows_vofs(int row, int chunk) {
+  const int odd = chunk & 1, slot = chunk >> 1;
+  return row * kRowBf16Bytes + 512 * odd + 256 * (slot >> 4) + 16 * ((slot & 15) ^ rows_f(row) ^ (4 * odd));
+}
+
+// n / d for 0 <= n < 2^31 by the host's multiplier (div_magic).
+struct Div {
+  uint32_t mul;
+  int sh;      // -1: d == 1
+};
+__device__ __forceinline__ int fast_div(int n, const Div d) {
+  const uint32_t q = __umulhi(static_cast<uint32_t>(n), d.mul) >> (d.sh & 31);
+  return d.sh < 0 ? n : static_cast<int>(q);
+}
+
+__device__ __forceinline__ float lane_read(int byte_addr, float v) {
+  return __uint_as_float(static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(byte_addr, static_cast<int>(__float_as_uint(v)))));
+}
+
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+template <int kMode, int kW>
+__global__ __launch_bounds__(64 * kW) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void sparse_mla_rows_kernel(const MlaArgs a, const Div block_div, const Div pool_div) {
+  constexpr bool kPaged = kMode != kFlatRows;
+  constexpr int kUnit = 16 * kW;              // keys per unit
+  constexpr int kTiles = 32 / kW;             // 16-latent output tiles of a wave
+  __shared__ RowsShared<kW> sh;
+  const int split = blockIdx.x, t = blockIdx.y, hg = blockIdx.z;
+  const int w = uniform(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int g = lane >> 4;
+  const int c = lane & 15;
+  const int start = split * a.split_len;
+  const int end = min(start + a.split_len, a.topk);
+  const int units = end > start ? (end - start + kUnit - 1) / kUnit : 0;
+  const int head = hg * kHeads + c;
+  const bool head_ok = head < a.num_heads;
+  const int32_t* idx_t = a.idx + t * a.si_t;
+  const int req = kPaged ? a.req_id[t] : 0;
+  const bool req_ok = kPaged && req >= 0 && req < a.num_reqs && a.max_blocks > 0;
+  const int32_t* bt_req = !kPaged ? nullptr : req_ok ? a.bt + static_cast<int64_t>(req) * a.bt_stride : a.req_id + t;
+  const int max_blocks = req_ok ? a.max_blocks : 0;
+  const int last_blk = max(max_blocks, 1) - 1;
+  const int32_t* pools_t = kMode != kPooledPos ? nullptr : a.num_pools > 0 ? a.pools + t * a.sp_t : a.req_id + t;
+  const int last_pool = max(a.num_pools, 1) - 1;
+  const int seq_len_t = kMode == kPooledPos && a.seq_lens ? a.seq_lens[t] : -1;
+  const int tail0 = seq_len_t >= 0 ? fast_div(seq_len_t, pool_div) * a.pool_size : 0;
+  uint8_t* vb = reinterpret_cast<uint8_t*>(&sh.v[0][0]);
+  // this lane's place in rows 16 w + 2 i + lane / 32: 16 codes, chunks 2 p and 2 p + 1, p = lane % 32
+  const int wr_half = (16 * w + (lane >> 5)) * kRowBf16Bytes + 256 * ((lane >> 4) & 1);
+  const int wr_low = 16 * ((lane & 15) ^ (lane >> 5));
+  const int k_base = rows_vofs(16 * w + c, g);
+  // rows 4 g + c / 4 (+ 16 per wave), latents (512 / kW) w + 16 dt + 4 (c % 4) + [0, 4)
+  const int tr_slot = 32 / kW * w;
+  const int tr_base = (rows_vofs(4 * g + (c >> 2), (c & 3) >> 1) + 8 * (c & 1) + 256 * (tr_slot >> 4)) ^ (16 * (tr_slot & 15));
+
+  // A negative softmax scale is moved into q (exact), so that the maximum
+  // is taken on q . k * row scale; zero counts as the smallest positive scale
+  // (every weight 1).
+  const float cs = fmaxf(fabsf(a.scale_log2), 1.0e-37f);
+  const uint32_t flip = a.scale_log2 < 0.f ? 0x80008000u : 0u;
+  bf16x8 qf[16];
+  {
+    const uint4* qp = reinterpret_cast<const uint4*>(a.q + t * a.sq_t + (head_ok ? head : 0) * a.sq_h + 8 * g);
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+      uint4 v = qp[4 * i];
+      v = make_uint4(v.x ^ flip, v.y ^ flip, v.z ^ flip, v.w ^ flip);
+      qf[i] = __builtin_bit_cast(bf16x8, head_ok ? v : make_uint4(0, 0, 0, 0));
+    }
+  }
+
+  f32x4 acc[kTiles];
+#pragma unroll
+  for (int i = 0; i < kTiles; i++) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float mc = kNegLarge * cs, l_run = 0.f;   // running maximum (base-2 logit units); l: this wave's keys only
+
+  auto key_pos = [&](int n) { return start + n * kUnit + 16 * w + c; };
+  auto load_raw = [&](int n) {
+    const int k = min(key_pos(n), end - 1);
+    if constexpr (kMode == kPooledPos) return pools_t[min(fast_div(k, pool_div), last_pool)];
+    else return idx_t[k];
+  };
+  struct Look {
+    int e;     // flat: the row or -1; paged: the block-table entry
+    int rel;   // paged: the row within its page, or -1 for a masked key
+  };
+  auto lookup = [&](int raw, int n) {
+    const int pos = key_pos(n);
+    Look l;
+    if constexpr (kMode == kFlatRows) {
+      l.e = pos < end && raw >= 0 && static_cast<int64_t>(raw) < a.seq_kv ? raw : -1;
+      l.rel = 0;
+    } else {
+      int p = raw;
+      if constexpr (kMode == kPooledPos) {
+        const int expanded = a.num_pools * a.pool_size;
+        const int j = pos - expanded;
+        const int pq = fast_div(pos, pool_div);
+        p = pos < expanded ? (raw >= 0 ? raw * a.pool_size + (pos - pq * a.pool_size) : -1)
+            : seq_len_t >= 0 && j < a.pool_size - 1 && j < seq_len_t - tail0 ? tail0 + j : -1;
+      }
+      const int blk = fast_div(max(p, 0), block_div);
+      l.e = bt_req[min(blk, last_blk)];
+      l.rel = pos < end && p >= 0 && blk < max_blocks ? p - blk * a.block_size : -1;
+    }
+    return l;
+  };
+  // The rows in 16-byte units of the cache (the host keeps them below 2^32).
+  uint4 d[8];           // codes 16 (lane % 32) + [0, 16) of key 2 i + lane / 32
+  float sv = 0.f;       // scale of key c (garbage for a masked key)
+  uint32_t vmask = 0;   // bit c: key c valid
+  const uint8_t* kv_lane = a.kv + 16 * (lane & 31);
+  auto issue_rows = [&](const Look& l) {
+    const bool ok = kPaged ? l.rel >= 0 && l.e >= 0 && l.e < a.num_blocks : l.e >= 0;
+    uint32_t u = kPaged ? static_cast<uint32_t>(l.e) * static_cast<uint32_t>(a.page_units) +
+                              static_cast<uint32_t>(l.rel) * static_cast<uint32_t>(a.row_units)
+                        : static_cast<uint32_t>(l.e) * static_cast<uint32_t>(a.row_units);
+    u = ok ? u : 0u;
+    vmask = static_cast<uint32_t>(__ballot(ok)) & 0xffffu;
+    sv = *reinterpret_cast<const float*>(a.kv + static_cast<uint64_t>(u) * 16 + kLatent);
+    int ka = 4 * (lane >> 5);
+    asm("" : "+v"(ka));   // one address register, the keys as immediate offsets
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      const uint32_t ui = static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(ka + 8 * i, static_cast<int>(u)));
+      d[i] = *reinterpret_cast<const uint4*>(kv_lane + static_cast<uint64_t>(ui) * 16);
+    }
+  };
+
+  int raw = -1;
+  Look look = {-1, -1};
+  if (units > 0) {
+    const int i0 = load_raw(0), i1 = load_raw(1);
+    raw = load_raw(2);
+    const Look k0 = lookup(i0, 0);
+    look = lookup(i1, 1);
+    issue_rows(k0);
+  }
+#pragma clang loop unroll(disable)
+  for (int n = 0; n < units; n++) {
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      bf16x8 lo, hi;
+      i8x16_to_bf16(d[i], lo, hi);
+      // chunks 2 p and 2 p + 1 of row 16 w + 2 i + lane / 32 (rows_f is linear in the row's bits)
+      uint8_t* row = vb + wr_half + 2 * i * kRowBf16Bytes;
+      *reinterpret_cast<bf16x8*>(row + (wr_low ^ (16 * rows_f(2 * i)))) = lo;
+      *reinterpret_cast<bf16x8*>(row + (wr_low ^ (16 * rows_f(2 * i)) ^ 64) + 512) = hi;
+    }
+    const float svm = (vmask >> c) & 1 ? sv : 0.f;
+    const uint32_t valid = vmask;
+    float sc[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++) sc[r] = lane_read(16 * g + 4 * r, svm);
+    __builtin_amdgcn_sched_barrier(0);
+    issue_rows(look);
+    look = lookup(raw, n + 2);
+    raw = load_raw(n + 3);
+    __builtin_amdgcn_sched_barrier(0);
+
+    f32x4 sacc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+      // chunk 4 i + g: place 2 i + g / 2 of its half
+      const bf16x8 k = *reinterpret_cast<const bf16x8*>(vb + (k_base ^ (32 * (i & 7))) + 256 * (i >> 3));
+      sacc[i & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k, qf[i], sacc[i & 1], 0, 0, 0);
+    }
+    float s[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++) s[r] = (sacc[0][r] + sacc[1][r]) * sc[r];
+    if (valid != 0xffffu) {   // uniform: a masked key
+#pragma unroll
+      for (int r = 0; r < 4; r++) s[r] = (valid >> (4 * g + r)) & 1 ? s[r] : -__builtin_inff();
+    }
+    float pr[4];
+    auto weights = [&]() {
+#pragma unroll
+      for (int r = 0; r < 4; r++) pr[r] = fast_exp2(__builtin_fmaf(s[r], cs, -mc));
+      sh.p[w][lane] = make_uint2(pack_bf16x2(pr[0] * sc[0], pr[1] * sc[1]), pack_bf16x2(pr[2] * sc[2], pr[3] * sc[3]));
+    };
+    weights();
+    const float mx = rows_max(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])));
+    if (g == 0) sh.mx[c][w] = mx;
+    lds_barrier();   // the unit's rows, weights and maxima are in LDS
+    float m_all = sh.mx[c][0];
+#pragma unroll
+    for (int i = 1; i < kW; i++) m_all = fmaxf(m_all, sh.mx[c][i]);
+    // every wave sees the same maxima, so all take the same branch
+    if (__ballot(m_all * cs > mc)) {
+      const float mc_new = fmaxf(mc, m_all * cs);
+      const float alpha = fast_exp2(mc - mc_new);
+      mc = mc_new;
+      l_run *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < kTiles; dt++) {
+        acc[dt][0] *= alpha; acc[dt][1] *= alpha; acc[dt][2] *= alpha; acc[dt][3] *= alpha;
+      }
+      weights();
+      lds_barrier();
+    }
+    bf16x8 pb[kW / 2];
+#pragma unroll
+    for (int h = 0; h < kW / 2; h++) {
+      const uint2 x = sh.p[2 * h][lane], y = sh.p[2 * h + 1][lane];
+      pb[h] = __builtin_bit_cast(bf16x8, make_uint4(x.x, x.y, y.x, y.y));
+    }
+#pragma unroll
+    for (int dt = 0; dt < kTiles; dt++) {
+      const uint8_t* vt = vb + (tr_base ^ (16 * (dt & 15)));
+#pragma unroll
+      for (int h = 0; h < kW / 2; h++) {
+        const i16x4 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(GLM53_LDS(i16x4, vt + 32 * h * kRowBf16Bytes));
+        const i16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(GLM53_LDS(i16x4, vt + (32 * h + 16) * kRowBf16Bytes));
+        const i32x2 v0i = __builtin_bit_cast(i32x2, v0);
+        const i32x2 v1i = __builtin_bit_cast(i32x2, v1);
+        const uint4 vv = make_uint4(v0i[0], v0i[1], v1i[0], v1i[1]);
+        acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, vv), pb[h], acc[dt], 0, 0, 0);
+      }
+    }
+    l_run += rows_sum((pr[0] + pr[1]) + (pr[2] + pr[3]));
+    lds_barrier();   // every wave has read the unit's rows
+  }
+
+  // the waves' shares of the denominator, in wave order
+  if (g == 0) sh.mx[c][w] = l_run;
+  lds_barrier();
+  float l = sh.mx[c][0];
+#pragma unroll
+  for (int i = 1; i < kW; i++) l += sh.mx[c][i];
+  const float inv_l = 1.f / (l > 0.f ? l : 1.f);
+  const int tile0 = kTiles * w;   // first 16-latent tile of this wave
+  if (a.num_splits == 1 && !a.partials_only) {
+    if (!head_ok) return;
+    uint16_t* op = a.out + t * a.so_t + head * a.so_h + 16 * tile0 + 4 * g;
+#pragma unroll
+    for (int dt = 0; dt < kTiles; dt++)
+      *reinterpret_cast<uint2*>(op + 16 * dt) = make_uint2(pack_bf16x2(acc[dt][0] * inv_l, acc[dt][1] * inv_l),
+                                                           pack_bf16x2(acc[dt][2] * inv_l, acc[dt][3] * inv_l));
+  } else {
+#pragma unroll
+    for (int dt = 0; dt < kTiles; dt++)
+      store_through(part_block(a, t, split, hg), ((tile0 + dt) * 64 + lane) * 16,
+                    make_float4(acc[dt][0] * inv_l, acc[dt][1] * inv_l, acc[dt][2] * inv_l, acc[dt][3] * inv_l));
+    if (w == 0 && g == 0 && head_ok)
+      a.lse[(static_cast<int64_t>(t) * a.num_splits + split) * a.heads_padded + head] = (mc + log2f(l)) * kLn2;
+  }
+}
+
 // ---------------------------------------------------------------- gather floor (diagnostic)
 // The memory chain of sparse_mla_kernel's decode splits alone: the same grid
 // and workgroup shape, the same index loads, row gathers and scale loads per
@@ -1216,6 +1520,57 @@ __global__ __launch_bounds__(kMergeThreads) void sparse_mla_merge_kernel(const f
   }
 }
 
+// The merge of at most kFewSplits splits: one wave per (token, head group,
+// 16-latent tile), every split's block and LSE of the tile in flight at once,
+// the same sums in the same order as sparse_mla_merge_kernel (whose split
+// lanes hold one split each then) with no LDS and no barrier.
+constexpr int kFewSplits = 8;
+constexpr int kFewThreads = 256;
+
+__global__ __launch_bounds__(kFewThreads) void sparse_mla_merge_few_kernel(const float* __restrict__ part,
+                                                                           const float* __restrict__ lse,
+                                                                           int num_splits, int heads_padded,
+                                                                           int num_heads, uint16_t* __restrict__ out,
+                                                                           int64_t so_t, int64_t so_h) {
+  const int groups = heads_padded / kHeads;
+  const int t = blockIdx.x / groups, hg = blockIdx.x % groups;
+  const int tile = blockIdx.y * (kFewThreads / 64) + uniform(threadIdx.x >> 6);
+  const int p = threadIdx.x & 63;
+  const int head = hg * kHeads + (p & 15);
+  const int64_t blk_stride = static_cast<int64_t>(groups) * kHeads * kLatent;
+  const float* pp = part + (static_cast<int64_t>(t) * num_splits * groups + hg) * kHeads * kLatent + (tile * 64 + p) * 4;
+  const float* lp = lse + static_cast<int64_t>(t) * num_splits * heads_padded + head;
+  f32x4 pv[kFewSplits];
+  float lv[kFewSplits];
+#pragma unroll
+  for (int s = 0; s < kFewSplits; s++) {
+    pv[s] = f32x4{0.f, 0.f, 0.f, 0.f};
+    lv[s] = kNegLarge;
+    if (s < num_splits) {   // uniform; read once: streaming loads
+      pv[s] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(pp + s * blk_stride));
+      lv[s] = lp[static_cast<int64_t>(s) * heads_padded];
+    }
+  }
+  float m = kNegLarge;
+#pragma unroll
+  for (int s = 0; s < kFewSplits; s++) m = fmaxf(m, lv[s]);
+  f32x4 r = f32x4{0.f, 0.f, 0.f, 0.f};
+  float den = 0.f;
+#pragma unroll
+  for (int s = 0; s < kFewSplits; s++) {
+    if (s < num_splits) {
+      const float e = expf(lv[s] - m);
+      r += f32x4{e * pv[s][0], e * pv[s][1], e * pv[s][2], e * pv[s][3]};
+      den += e;
+    }
+  }
+  if (head >= num_heads) return;
+  const float inv = 1.f / (den > 0.f ? den : 1.f);
+  const int d = 16 * tile + 4 * (p >> 4);
+  *reinterpret_cast<uint2*>(out + t * so_t + head * so_h + d) =
+      make_uint2(pack_bf16x2(r[0] * inv, r[1] * inv), pack_bf16x2(r[2] * inv, r[3] * inv));
+}
+
 }  // namespace
 }  // namespace glm53
 
@@ -1292,6 +1647,51 @@ int64_t tokens_grid(int64_t num_tokens, int heads_padded, int64_t num_splits) {
   return num_splits <= 32 * (8 / tp) ? tp : num_tokens;   // each XCD's share within its 32 CUs
 }
 
+// Compute units of the current device (looked up once per device).
+int num_cus() {
+  static std::atomic<int> cached[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  int n = cached[dev].load(std::memory_order_relaxed);
+  if (!n) {
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1) n = 256;
+    cached[dev].store(n, std::memory_order_relaxed);
+  }
+  return n;
+}
+
+// Multiplier of fast_div: n / d = mulhi(n, mul) >> sh for 0 <= n < 2^31.  With
+// 2^(s-1) < d <= 2^s and mul = floor(2^(31+s) / d) + 1 (below 2^32), mul * d
+// exceeds 2^(31+s) by at most d <= 2^s, so n * (mul * d - 2^(31+s)) < 2^(31+s)
+// and the quotient is exact.
+Div div_magic(int64_t d) {
+  if (d <= 1) return Div{0u, -1};
+  int s = 0;
+  while ((int64_t(1) << s) < d) s++;
+  return Div{static_cast<uint32_t>((uint64_t(1) << (31 + s)) / static_cast<uint64_t>(d) + 1), s - 1};
+}
+
+// Waves per workgroup of sparse_mla_rows_kernel for a long split, or 0 for
+// the pair kernel.  A compute unit holds one workgroup of 8 waves or two of 4
+// (a round of the former takes 51-57 us at 2176 keys, of the latter 62-66 with
+// one per CU and 90-107 with two): 8 waves where they need one round, or three
+// against the 4-wave form's half-filled second (640 workgroups 154 us against
+// 158, 700 156 / 163), but not for a few units (splits of 436 and 544 keys: 23.8
+// / 22.4 and 27.0 / 25.9 us at 48 and 64 tokens).  From three to three and a
+// half rounds the pair kernel, four workgroups to a CU, is still ahead (800:
+// 174 us against 183; 900: 189 / 188).  Row offsets are 32-bit counts of 16
+// bytes here; a flat cache that spans more keeps the pair kernel's 64 bits.
+int rows_waves(const MlaArgs& a, int mode, int64_t workgroups) {
+  if (mode == kFlatRows && (a.skv < 0 || (a.seq_kv - 1) > int64_t(0xffffffff) / (a.skv / 16 > 0 ? a.skv / 16 : 1)))
+    return 0;
+  const int64_t cus = num_cus();
+  if (workgroups <= cus) return a.split_len >= 640 ? 8 : 4;
+  if (workgroups <= 2 * cus) return 4;
+  if (workgroups <= 3 * cus) return 8;
+  if (2 * workgroups <= 7 * cus) return 0;
+  return 4;
+}
+
 void launch_attention(const MlaArgs& a, int64_t num_tokens, hipStream_t st) {
   // Splits longer than one chunk of gathers pipeline their chunks.
   const bool pipe = a.split_len > kChunkTiles * kTile;
@@ -1327,6 +1727,23 @@ void launch_attention(const MlaArgs& a, int64_t num_tokens, hipStream_t st) {
       hipLaunchKernelGGL((sparse_mla_kernel<M, false, G>), grid, dim3(SplitShape<G>::kThreads), 0, st,       \
                          GLM53_LEAD);                                                                  \
   } while (0)
+  if (const int waves = pair ? rows_waves(a, mode, static_cast<int64_t>(grid.x) * grid.y * grid.z) : 0) {
+    MlaArgs ra = a;
+    if (mode == kFlatRows) ra.row_units = static_cast<int>(static_cast<uint32_t>(a.skv / 16));
+    const Div bd = div_magic(a.block_size), pd = div_magic(a.pool_size);
+#define GLM53_ROWS(M)                                                                                           \
+  do {                                                                                                          \
+    if (waves == 8)                                                                                             \
+      hipLaunchKernelGGL((sparse_mla_rows_kernel<M, 8>), grid, dim3(512), 0, st, ra, bd, pd);                   \
+    else                                                                                                        \
+      hipLaunchKernelGGL((sparse_mla_rows_kernel<M, 4>), grid, dim3(256), 0, st, ra, bd, pd);                   \
+  } while (0)
+    if (mode == kPooledPos) GLM53_ROWS(kPooledPos);
+    else if (mode == kPagedPos) GLM53_ROWS(kPagedPos);
+    else GLM53_ROWS(kFlatRows);
+#undef GLM53_ROWS
+    return;
+  }
   if (mode == kPooledPos) {
     if (pair) GLM53_PAIR(kPooledPos); else if (pipe) GLM53_LAUNCH(kPooledPos, true);
     else if (three) GLM53_KG(kPooledPos, 3); else if (one) GLM53_KG(kPooledPos, 1); else GLM53_LAUNCH(kPooledPos, false);
@@ -1346,6 +1763,15 @@ void launch_attention(const MlaArgs& a, int64_t num_tokens, hipStream_t st) {
 void launch_merge(const float* part, const float* lse, int64_t num_tokens, int num_splits,
                   int heads_padded, int num_heads, uint16_t* out, int64_t so_t, int64_t so_h,
                   hipStream_t st) {
+  // Few splits of many (token, head group) units: the 512-thread workgroups
+  // of the other form have a wave per split lane, most of them idle (48 tokens
+  // of 5 splits 9.8 -> 3.5 us, 64 of 4 and 128 of 2 alike).
+  if (num_splits <= kFewSplits && num_tokens * (heads_padded / kHeads) >= 16) {
+    hipLaunchKernelGGL(sparse_mla_merge_few_kernel,
+                       dim3(static_cast<unsigned>(num_tokens * (heads_padded / kHeads)), 32 / (kFewThreads / 64)),
+                       dim3(kFewThreads), 0, st, part, lse, num_splits, heads_padded, num_heads, out, so_t, so_h);
+    return;
+  }
   const int64_t tg = tokens_grid(num_tokens, heads_padded, num_splits);
   const dim3 grid(static_cast<unsigned>(tg * (heads_padded / kHeads)), 32);
   if (tg != num_tokens)

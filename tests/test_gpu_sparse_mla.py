@@ -608,3 +608,64 @@ def test_long_split_pair_kernel_edges(cuda, oracle, small_cache):
     out = triton_mla_sparse_attention(q, empty, idx, W.SM_SCALE, num_kv_splits=1)
     torch.cuda.synchronize()
     assert torch.equal(out, torch.zeros_like(out))
+
+
+@pytest.mark.parametrize("T,H,topk,splits", [
+    (3, 16, 288, 1), (2, 20, 320, 1), (48, 16, 2176, 5), (12, 80, 2176, 8), (28, 80, 2176, 8),   # 64-key units
+    (2, 16, 640, 1), (3, 8, 672, 1), (5, 32, 2176, 2), (20, 80, 2176, 6),                         # 128-key units
+    (20, 80, 2176, 8)])                                                                           # the pair kernel
+def test_long_split_rows_kernel_edges(cuda, oracle, small_cache, T, H, topk, splits):
+    """Splits of more than 256 keys in units of 64 or 128 keys: the last unit
+    whole, half or a few keys, the first half of a row's indices masked (whole
+    masked units before and after the first valid one), indices outside the
+    cache both ways, 1 to 5 head groups with a padded one, 1 to 8 splits
+    through either merge, and the grids on both sides of each step of the
+    kernel choice; the paged form is bit-identical."""
+    from titan_mla import triton_mla_sparse_attention, triton_mla_sparse_attention_paged
+    w, rows = small_cache
+    n = w["n_rows"]
+    kv = w["cache"].view(n, 1, 528)
+    g = W.gen(cuda, 1000 + topk + T)
+    q = torch.randn(T, H, 512, generator=g, device=cuda).to(torch.bfloat16)
+    idx = torch.randint(-40, n + 40, (T, 1, topk), generator=g, device=cuda, dtype=torch.int32)
+    idx[0, :, topk // 2:] = -1
+    idx[1, :, :topk // 2] = -1
+    log_case("mla rows kernel", T, H, topk, splits)
+    out = triton_mla_sparse_attention(q, kv, idx, W.SM_SCALE, num_kv_splits=splits)
+    torch.cuda.synchronize()
+    want = oracle.sparse_mla(u16(q), rows, idx.cpu().numpy(), W.SM_SCALE, n_splits=splits, groups=1, block_n=32)
+    compare(out, want, ("rows kernel", T, H, topk, splits))
+    blank = triton_mla_sparse_attention(q, kv, torch.full_like(idx, -1), W.SM_SCALE, num_kv_splits=splits)
+    assert torch.equal(blank, torch.zeros_like(blank))
+    pages = w["cache"].view(n // 64, 64, 528)
+    table = torch.arange(n // 64, device=cuda, dtype=torch.int32)[None, :]
+    req = torch.zeros(T, dtype=torch.int32, device=cuda)
+    paged = triton_mla_sparse_attention_paged(q, pages, idx, req, table, W.SM_SCALE, num_kv_splits=splits)
+    torch.cuda.synchronize()
+    assert torch.equal(paged, out)
+
+
+@pytest.mark.parametrize("topk", [288, 1088])
+@pytest.mark.parametrize("sm_scale", [W.SM_SCALE, -W.SM_SCALE, 0.0])
+@pytest.mark.parametrize("order", ["rising", "falling", "late"])
+def test_long_split_running_maximum(cuda, topk, sm_scale, order):
+    """Weights are computed against the maximum of the units before and again
+    where a unit raises it: the spread of the logits rises or falls over the
+    split (row scales), or steps up at a late unit, with either sign of the
+    softmax scale and zero, against float64."""
+    from titan_mla import triton_mla_sparse_attention
+    g = W.gen(cuda, 77)
+    cache = torch.zeros(topk, 528, dtype=torch.int8, device=cuda)
+    cache[:, :512] = torch.randint(-127, 128, (topk, 512), generator=g, device=cuda, dtype=torch.int8)
+    ramp = torch.arange(topk, device=cuda, dtype=torch.float32) / topk
+    scale = {"rising": 0.02 + ramp, "falling": 1.02 - ramp, "late": torch.where(ramp > 0.9, 0.06, 0.03)}[order]
+    cache[:, 512:516] = scale.float().view(torch.int8).view(topk, 4)
+    q = torch.randn(2, 16, 512, generator=g, device=cuda).to(torch.bfloat16)
+    idx = torch.arange(topk, device=cuda, dtype=torch.int32).expand(2, 1, topk).contiguous()
+    log_case("mla running maximum", topk, sm_scale, order)
+    out = triton_mla_sparse_attention(q, cache.view(topk, 1, 528), idx, sm_scale, num_kv_splits=1)
+    torch.cuda.synchronize()
+    k = cache[:, :512].double().cpu().numpy() * scale.double().cpu().numpy()[:, None]
+    logits = np.einsum("thd,kd->thk", q.double().cpu().numpy(), k) * sm_scale
+    p = np.exp(logits - logits.max(-1, keepdims=True))
+    textbook_check(out, np.einsum("thk,kd->thd", p / p.sum(-1, keepdims=True), k), (topk, sm_scale, order))
