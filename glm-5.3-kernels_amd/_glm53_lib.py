@@ -34,8 +34,10 @@ EXPORTED = (
     "glm53_fused_moe_w4a16_workspace_bytes",
     "glm53_fused_moe_w4a16",
     "glm53_fp8_paged_mqa_logits",
+    "glm53_fp8_paged_mqa_logits_next_n",
     "glm53_indexer_topk_workspace_bytes",
     "glm53_indexer_topk",
+    "glm53_indexer_topk_next_n",
     "glm53_stream_probe",
 )
 
@@ -103,10 +105,15 @@ def load():
     L.glm53_fp8_paged_mqa_logits.restype = I
     L.glm53_fp8_paged_mqa_logits.argtypes = [P, I64, I64, P, I64, I64, I64, P, I64, P, P, I64, I64, I64, I64,
                                              I64, I64, I, P, I64, P]
+    L.glm53_fp8_paged_mqa_logits_next_n.restype = I
+    L.glm53_fp8_paged_mqa_logits_next_n.argtypes = [P, I64, I64, P, I64, I64, I64, P, I64, P, P, I64, I64, I64, I64,
+                                                    I64, I64, I64, I, P, I64, P]
     L.glm53_indexer_topk_workspace_bytes.restype = I64
     L.glm53_indexer_topk_workspace_bytes.argtypes = [I64, I64, I64]
     L.glm53_indexer_topk.restype = I
     L.glm53_indexer_topk.argtypes = [P, I64, P, I64, I64, I64, P, I64, P, I64, P]
+    L.glm53_indexer_topk_next_n.restype = I
+    L.glm53_indexer_topk_next_n.argtypes = [P, I64, P, I64, I64, I64, I64, P, I64, P, I64, P]
     L.glm53_stream_probe.restype = I
     L.glm53_stream_probe.argtypes = [I, P, P, I64, P]
     version = L.glm53_abi_version()

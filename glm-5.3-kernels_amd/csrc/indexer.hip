@@ -76,7 +76,15 @@ struct LogitsArgs {
   float* logits;            // [T][max_len], row stride sl_t
   int64_t sl_t;
   int clean;                // write -inf at positions >= context length
+  int next_n;               // query rows per request (kRows > 1)
+  int row_blocks;           // workgroup rows per request: ceil(next_n / kRows)
 };
+
+// Context length of query row i of n of a request whose last row sees ctx
+// positions (32-bit arithmetic wraps).
+__device__ __forceinline__ int query_len(int ctx, int n, int i) {
+  return static_cast<int>(static_cast<uint32_t>(ctx) - static_cast<uint32_t>(n - 1 - i));
+}
 
 __device__ __forceinline__ float row_sum4(float v) {
   // sum over lanes l, l^16, l^32, l^48 (the four 16-lane rows)
@@ -176,20 +184,30 @@ __device__ __forceinline__ void load_group(const LogitsArgs& a, int t, int j0, i
   gr.sc = *reinterpret_cast<const float*>(page + static_cast<int64_t>(a.block_size) * kHeadDim + 4 * off);
 }
 
-// Wave = a run of kN 16-key groups of one token's row; the block-table
-// entries of all its groups are read at once (lane i: group i), then the
-// groups stream through a kDepth-deep ring of register slots, the loads of
-// group i + kDepth - 1 issued before group i is reduced, so each wave keeps
-// kDepth - 1 groups (6 KB at depth 4) in flight.  The run is unrolled
+// Wave = a run of kN 16-key groups of kRows query rows of one request; the
+// block-table entries of all its groups are read at once (lane i: group i),
+// then the groups stream through a kDepth-deep ring of register slots, the
+// loads of group i + kDepth - 1 issued before group i is reduced, so each wave
+// keeps kDepth - 1 groups (6 KB at depth 4) in flight.  The run is unrolled
 // whole and its loads issued on every path, and the results wait in LDS
 // for stores after the last load (stores count with the loads in vmcnt):
 // every wait then counts exactly the group it needs.
-template <int kTiles, int kN, bool kAligned>
+//
+// Decode: the request's one row.  kSpec: the next_n rows of a
+// speculative step, which differ in their last few positions only: a group is
+// loaded once for up to kRows of them (the loads set the time: one L1 access
+// per 16 bytes of a key), each row's results end at its own length.
+// 24 requests x 12000 keys, 32 heads: 2 rows 16.7 -> 13.3 us, 4 rows 24.9 -> 19.4.
+// kSpec alone (kRows = 1): the rows one by one.
+template <int kTiles, int kN, bool kAligned, int kRows, bool kSpec>
 __global__ __launch_bounds__(kLogitThreads) void fp8_paged_mqa_logits_kernel(
     const int32_t* ctx, const int32_t* bt, int64_t bt_stride, const uint8_t* q, int64_t sq_t, int keys_per_wg,
     int max_len, int block_size, int max_blocks, const LogitsArgs a) {
   constexpr int kDepth = 4;
-  const int t = blockIdx.y;
+  const int req = !kSpec ? blockIdx.y : blockIdx.y / a.row_blocks;
+  const int first = !kSpec ? 0 : (blockIdx.y - req * a.row_blocks) * kRows;   // of the request's rows
+  const int rows = kRows == 1 ? 1 : min(kRows, a.next_n - first);
+  const int t0 = !kSpec ? req : req * a.next_n + first;
   const int lane = threadIdx.x & 63;
   const int w = uniform(threadIdx.x >> 6);
   const int g = lane >> 4, c = lane & 15;
@@ -198,39 +216,49 @@ __global__ __launch_bounds__(kLogitThreads) void fp8_paged_mqa_logits_kernel(
   if (j_wave >= j_end) return;   // uniform (no barriers in this kernel)
   const int n = (j_end - j_wave + 15) / 16;
   const int cap = max_blocks * block_size;
-  int len = ctx[t];
-  len = len < 0 ? 0 : len > cap ? cap : len;
+  const int ctx_t = ctx[req];
+  auto row_len = [&](int r) {
+    const int l = !kSpec ? ctx_t : query_len(ctx_t, a.next_n, first + r);
+    return l < 0 ? 0 : l > cap ? cap : l;
+  };
+  int len = row_len(0);   // the longest row's
+#pragma unroll
+  for (int r = 1; r < kRows; r++)
+    if (r < rows) len = max(len, row_len(r));
 
   // page of each group's first key (lane i < n: group i; -1 past the context)
   int blk_l = -1;
   if (lane < n) {
     const int j0 = j_wave + 16 * lane;
-    if (j0 < len) blk_l = bt[t * bt_stride + j0 / block_size];
+    if (j0 < len) blk_l = bt[req * bt_stride + j0 / block_size];
   }
 
   // q fragments (A operand) and the weights of this lane's heads.
-  uint64_t qf[kTiles][4];
-  float wv[kTiles][4];
+  uint64_t qf[kRows][kTiles][4];
+  float wv[kRows][kTiles][4];
 #pragma unroll
-  for (int ht = 0; ht < kTiles; ht++) {
-    const uint4* qp = reinterpret_cast<const uint4*>(q + t * sq_t + (16 * ht + c) * a.sq_h + 16 * g);
-    const uint4 lo = qp[0], hi = qp[4];
-    qf[ht][0] = (static_cast<uint64_t>(lo.y) << 32) | lo.x;
-    qf[ht][1] = (static_cast<uint64_t>(lo.w) << 32) | lo.z;
-    qf[ht][2] = (static_cast<uint64_t>(hi.y) << 32) | hi.x;
-    qf[ht][3] = (static_cast<uint64_t>(hi.w) << 32) | hi.z;
+  for (int r = 0; r < kRows; r++) {
+    const int t = t0 + min(r, rows - 1);
 #pragma unroll
-    for (int i = 0; i < 4; i++) wv[ht][i] = a.w[t * a.sw_t + 16 * ht + 4 * g + i];
+    for (int ht = 0; ht < kTiles; ht++) {
+      const uint4* qp = reinterpret_cast<const uint4*>(q + t * sq_t + (16 * ht + c) * a.sq_h + 16 * g);
+      const uint4 lo = qp[0], hi = qp[4];
+      qf[r][ht][0] = (static_cast<uint64_t>(lo.y) << 32) | lo.x;
+      qf[r][ht][1] = (static_cast<uint64_t>(lo.w) << 32) | lo.z;
+      qf[r][ht][2] = (static_cast<uint64_t>(hi.y) << 32) | hi.x;
+      qf[r][ht][3] = (static_cast<uint64_t>(hi.w) << 32) | hi.z;
+#pragma unroll
+      for (int i = 0; i < 4; i++) wv[r][ht][i] = a.w[t * a.sw_t + 16 * ht + 4 * g + i];
+    }
   }
 
-  float* out = a.logits + t * a.sl_t;
-  __shared__ float res[kLogitWaves][16 * kN];
+  __shared__ float res[kLogitWaves][kRows][16 * kN];
   Group ring[kDepth];
   // group i of the run, or past the run's end (a row's tail) its last group
   // again, loaded and not used
   auto load = [&](int i, Group& gr) {
     const int ic = i < n ? i : n - 1;
-    load_group<kAligned>(a, t, j_wave + 16 * ic, __builtin_amdgcn_readlane(blk_l, ic), len, g, c, gr);
+    load_group<kAligned>(a, req, j_wave + 16 * ic, __builtin_amdgcn_readlane(blk_l, ic), len, g, c, gr);
   };
 #pragma unroll
   for (int s = 0; s < kDepth - 1; s++)
@@ -241,34 +269,48 @@ __global__ __launch_bounds__(kLogitThreads) void fp8_paged_mqa_logits_kernel(
       if (i + kDepth - 1 < kN) load(i + kDepth - 1, ring[(i + kDepth - 1) % kDepth]);
       if (i >= n) continue;   // uniform (the tail of a row)
       const Group& gr = ring[i % kDepth];
-      float v = 0.f;
+      float v[kRows] = {};
       if (gr.live) {
         const uint64_t k0 = (static_cast<uint64_t>(gr.kd[0].y) << 32) | gr.kd[0].x;
         const uint64_t k1 = (static_cast<uint64_t>(gr.kd[0].w) << 32) | gr.kd[0].z;
         const uint64_t k2 = (static_cast<uint64_t>(gr.kd[1].y) << 32) | gr.kd[1].x;
         const uint64_t k3 = (static_cast<uint64_t>(gr.kd[1].w) << 32) | gr.kd[1].z;
         const i32x8 kb = signed_key(key_operand(k0, k1, k2, k3), gr.sc);
+        const float factor = key_factor(gr.sc);
 #pragma unroll
-        for (int ht = 0; ht < kTiles; ht++) {
-          const f32x4v d = dot128_fp8(qf[ht], kb);
+        for (int r = 0; r < kRows; r++) {
+          if (r >= rows) continue;   // uniform
 #pragma unroll
-          for (int e = 0; e < 4; e++) v = __builtin_fmaf(wv[ht][e], relu_dot(d[e]), v);
+          for (int ht = 0; ht < kTiles; ht++) {
+            const f32x4v d = dot128_fp8(qf[r][ht], kb);
+#pragma unroll
+            for (int e = 0; e < 4; e++) v[r] = __builtin_fmaf(wv[r][ht][e], relu_dot(d[e]), v[r]);
+          }
+          v[r] = factor * row_sum4(v[r]);
         }
-        v = key_factor(gr.sc) * row_sum4(v);
       }
       // page outside the cache, or past the context: -inf (written past the
       // context only when cleaning, which the stores below decide)
-      if (g == 0) res[w][16 * i + c] = gr.kok ? v : -__builtin_inff();
+#pragma unroll
+      for (int r = 0; r < kRows; r++)
+        if (g == 0) res[w][r][16 * i + c] = gr.kok ? v[r] : -__builtin_inff();
     }
   }
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
-  for (int r = 0; r < (16 * kN + 63) / 64; r++) {
-    const int idx = 64 * r + lane;
-    const int j = j_wave + idx;   // written inside the run, and past the context only when cleaning
-    if (idx < 16 * n && j < j_end && (j < len || a.clean)) out[j] = res[w][idx];
+  for (int o = 0; o < kRows; o++) {
+    if (o >= rows) continue;   // uniform
+    float* out = a.logits + (t0 + o) * a.sl_t;
+    const int row_end = row_len(o);
+#pragma unroll
+    for (int r = 0; r < (16 * kN + 63) / 64; r++) {
+      const int idx = 64 * r + lane;
+      const int j = j_wave + idx;   // written inside the run, and past the row's length only when cleaning
+      if (idx < 16 * n && j < j_end && (j < row_end || a.clean))
+        out[j] = !kSpec || j < row_end ? res[w][o][idx] : -__builtin_inff();
+    }
   }
 }
 
@@ -496,7 +538,7 @@ constexpr int kSweepKeys = 32;                      // keys per thread per sweep
 struct TopkArgs {
   const float* logits;      // [rows][*], row stride sl
   int64_t sl;
-  const int32_t* lengths;   // [rows] valid columns per row
+  const int32_t* lengths;   // [rows / next_n] valid columns of each request's last row
   int max_len;              // columns available in a row
   int k;
   int32_t* out;             // [rows][k], row stride so
@@ -506,6 +548,7 @@ struct TopkArgs {
   int chunks;
   int chunk_len;
   bool vec;                 // logits rows 16-byte aligned
+  int next_n;               // rows per request
 };
 
 // Order-preserving key: a larger float has a larger key; NaN -> 0, below
@@ -764,12 +807,13 @@ __device__ __forceinline__ void for_each_key(const uint32_t (&kk)[P], F&& f) {
   for (int j = 0; j < P; j++) f(kk[j]);
 }
 
-__device__ __forceinline__ int clamp_len(const int32_t* lengths, int max_len, int row) {
-  const int len = lengths[row];
+// Valid columns of a row: its own entry, or of a request's n rows the last
+// one's less the rows after it.
+__device__ __forceinline__ int clamp_len(const int32_t* lengths, int max_len, int row, int n) {
+  const int req = n == 1 ? row : row / n;
+  const int len = query_len(lengths[req], n, row - req * n);
   return len < 0 ? 0 : len > max_len ? max_len : len;
 }
-
-__device__ __forceinline__ int clamp_len(const TopkArgs& a, int row) { return clamp_len(a.lengths, a.max_len, row); }
 
 // Chunk stage: workgroup (row, chunk c) keeps the local top-k of positions
 // [c * chunk_len, (c + 1) * chunk_len) of the row, in position order, as
@@ -778,10 +822,10 @@ __device__ __forceinline__ int clamp_len(const TopkArgs& a, int row) { return cl
 template <int P, int kThreads>
 __global__ __launch_bounds__(kThreads) void topk_chunk_kernel(
     const float* p_logits, int64_t p_sl, const int32_t* p_lengths, int p_max_len, int p_k, int p_chunk_len,
-    int p_chunks, int p_vec, const TopkArgs a) {
+    int p_chunks, int p_vec, int p_next_n, const TopkArgs a) {
   __shared__ SelShared<kThreads> sh;
   const int row = blockIdx.x, c = blockIdx.y, tid = threadIdx.x;
-  const int len = clamp_len(p_lengths, p_max_len, row);
+  const int len = clamp_len(p_lengths, p_max_len, row, p_next_n);
   const int k = p_k;
   const int start = c * p_chunk_len;
   const int rest = len - start;
@@ -824,10 +868,10 @@ __global__ __launch_bounds__(kThreads) void topk_chunk_kernel(
 template <int P, bool kCand>
 __global__ __launch_bounds__(kFinalThreads) void topk_final_kernel(
     const int32_t* p_lengths, int p_max_len, int p_k, int p_chunks, uint32_t* p_cand_key, int32_t* p_cand_pos,
-    int32_t* p_out, int64_t p_so, int p_chunk_len, const TopkArgs a) {
+    int32_t* p_out, int64_t p_so, int p_chunk_len, int p_next_n, const TopkArgs a) {
   __shared__ SelShared<kFinalThreads> sh;
   const int row = blockIdx.x, tid = threadIdx.x;
-  const int len = clamp_len(p_lengths, p_max_len, row);
+  const int len = clamp_len(p_lengths, p_max_len, row, p_next_n);
   const int k = p_k;
   int32_t* out = p_out + row * p_so;
   if (len <= k) {   // every valid position is selected (uniform)
@@ -927,7 +971,7 @@ __device__ void sweep_row(SelShared<kThreads>& sh, const float* x, int len, int 
 __global__ __launch_bounds__(kSweepThreads) void topk_sweep_kernel(const TopkArgs a) {
   __shared__ SelShared<kSweepThreads> sh;
   const int row = blockIdx.x;
-  const int len = clamp_len(a, row);
+  const int len = clamp_len(a.lengths, a.max_len, row, a.next_n);
   const int k = a.k;
   int32_t* out = a.out + row * a.so;
   if (len <= k) {
@@ -963,7 +1007,7 @@ __device__ __forceinline__ float key_value(uint32_t key) {   // inverse of order
 template <int kThreads>
 __global__ __launch_bounds__(kThreads) void topk_row_kernel(
     const float* p_logits, int64_t p_sl, const int32_t* p_lengths, int p_max_len, int p_k, int p_vec,
-    int32_t* p_out, int64_t p_so) {
+    int32_t* p_out, int64_t p_so, int p_next_n) {
   constexpr int P = kListKeys / kThreads;      // list keys per thread
   constexpr int kRuns = P / 4;                 // sampled runs of 4 per thread
   constexpr int kVecs = 4;                     // 4-key loads per thread and step of the pass over the row
@@ -971,7 +1015,7 @@ __global__ __launch_bounds__(kThreads) void topk_row_kernel(
   __shared__ int32_t list[kListKeys];
   __shared__ uint32_t listed;
   const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
-  const int len = clamp_len(p_lengths, p_max_len, row);
+  const int len = clamp_len(p_lengths, p_max_len, row, p_next_n);
   const int k = p_k;
   const float* x = p_logits + row * p_sl;
   int32_t* out = p_out + row * p_so;
@@ -1202,36 +1246,52 @@ bool aligned(const void* p, uintptr_t n) { return (reinterpret_cast<uintptr_t>(p
 using LogitsKernel = void (*)(const int32_t*, const int32_t*, int64_t, const uint8_t*, int64_t, int, int, int, int,
                               LogitsArgs);
 
-template <int kTiles, bool kAligned>
+template <int kTiles, int kRows, bool kSpec>
 LogitsKernel pick_logits_n(int gpw) {
   switch (gpw) {
-    case 1: return fp8_paged_mqa_logits_kernel<kTiles, 1, kAligned>;
-    case 2: return fp8_paged_mqa_logits_kernel<kTiles, 2, kAligned>;
-    case 4: return fp8_paged_mqa_logits_kernel<kTiles, 4, kAligned>;
-    case 8: return fp8_paged_mqa_logits_kernel<kTiles, 8, kAligned>;
-    default: return fp8_paged_mqa_logits_kernel<kTiles, 16, kAligned>;
+    case 1: return fp8_paged_mqa_logits_kernel<kTiles, 1, true, kRows, kSpec>;
+    case 2: return fp8_paged_mqa_logits_kernel<kTiles, 2, true, kRows, kSpec>;
+    case 4: return fp8_paged_mqa_logits_kernel<kTiles, 4, true, kRows, kSpec>;
+    case 8: return fp8_paged_mqa_logits_kernel<kTiles, 8, true, kRows, kSpec>;
+    default: return fp8_paged_mqa_logits_kernel<kTiles, 16, true, kRows, kSpec>;
   }
 }
 
+// Rows of one request a workgroup scores.  Up to 32 heads the key loads set
+// the time and are shared by four rows where that fills a last workgroup
+// with three or four, else by two (24 requests x 12000 keys, 32 heads, one / two
+// / four rows, us: next_n 2 16.7 / 13.3 / 16.9, 3 20.9 / 20.6 / 18.3, 4 24.9 / 20.5
+// / 19.4, 5 29.0 / 24.5 / 28.0, 6 33.1 / 24.7 / 28.2).  With more heads the products
+// weigh as much and two rows' queries leave half the waves: pairs only for an
+// even next_n (64 heads, next_n 2 19.0 / 17.8, 3 24.1 / 26.1, 4 30.7 / 26.3) and
+// where the waves run through many groups (4 requests 7.3 / 9.5).
+int rows_per_wg(int64_t next_n, int tiles, bool al, int64_t request_groups) {
+  if (next_n == 1) return 1;
+  if (!al || tiles > 2) return next_n % 2 || request_groups < 8192 ? 1 : 2;
+  return (next_n + 1) % 4 <= 1 ? 4 : 2;
+}
+
+template <int kTiles>
+LogitsKernel pick_logits_rows(int gpw, int rows, bool spec, bool al) {
+  if (!al)
+    return !spec ? fp8_paged_mqa_logits_kernel<kTiles, 1, false, 1, false>
+                 : rows == 1 ? fp8_paged_mqa_logits_kernel<kTiles, 1, false, 1, true>
+                             : fp8_paged_mqa_logits_kernel<kTiles, 1, false, 2, true>;
+  if (!spec) return pick_logits_n<kTiles, 1, false>(gpw);
+  if (rows == 1) return pick_logits_n<kTiles, 1, true>(gpw);
+  if constexpr (kTiles <= 2)
+    if (rows == 4) return pick_logits_n<kTiles, 4, true>(gpw);
+  return pick_logits_n<kTiles, 2, true>(gpw);
+}
+
 // Kernel for 16 * tiles heads and gpw groups per wave (unaligned block
-// sizes: one group per wave only).
-template <bool kAligned>
-LogitsKernel pick_logits_kernel(int tiles, int gpw) {
-  if constexpr (kAligned) {
-    switch (tiles) {
-      case 1: return pick_logits_n<1, true>(gpw);
-      case 2: return pick_logits_n<2, true>(gpw);
-      case 3: return pick_logits_n<3, true>(gpw);
-      default: return pick_logits_n<4, true>(gpw);
-    }
-  } else {
-    (void)gpw;
-    switch (tiles) {
-      case 1: return fp8_paged_mqa_logits_kernel<1, 1, false>;
-      case 2: return fp8_paged_mqa_logits_kernel<2, 1, false>;
-      case 3: return fp8_paged_mqa_logits_kernel<3, 1, false>;
-      default: return fp8_paged_mqa_logits_kernel<4, 1, false>;
-    }
+// sizes: one group per wave).
+LogitsKernel pick_logits_kernel(int tiles, int gpw, int rows, bool spec, bool al) {
+  switch (tiles) {
+    case 1: return pick_logits_rows<1>(gpw, rows, spec, al);
+    case 2: return pick_logits_rows<2>(gpw, rows, spec, al);
+    case 3: return pick_logits_rows<3>(gpw, rows, spec, al);
+    default: return pick_logits_rows<4>(gpw, rows, spec, al);
   }
 }
 
@@ -1247,9 +1307,22 @@ extern "C" int glm53_fp8_paged_mqa_logits(const void* q, int64_t sq_t, int64_t s
                                           int64_t num_tokens, int64_t num_heads, int64_t head_dim,
                                           int64_t max_len, int clean_logits, float* logits, int64_t sl_t,
                                           void* stream) {
+  return glm53_fp8_paged_mqa_logits_next_n(q, sq_t, sq_h, kv_cache, page_bytes, block_size, num_blocks, weights,
+                                           sw_t, context_lens, block_table, bt_stride, max_blocks, num_tokens, 1,
+                                           num_heads, head_dim, max_len, clean_logits, logits, sl_t, stream);
+}
+
+extern "C" int glm53_fp8_paged_mqa_logits_next_n(const void* q, int64_t sq_t, int64_t sq_h, const void* kv_cache,
+                                                 int64_t page_bytes, int64_t block_size, int64_t num_blocks,
+                                                 const float* weights, int64_t sw_t, const int32_t* context_lens,
+                                                 const int32_t* block_table, int64_t bt_stride, int64_t max_blocks,
+                                                 int64_t num_requests, int64_t next_n, int64_t num_heads,
+                                                 int64_t head_dim, int64_t max_len, int clean_logits, float* logits,
+                                                 int64_t sl_t, void* stream) {
   if (!q || !kv_cache || !weights || !context_lens || !block_table || !logits) return GLM53_ERR_NULL_POINTER;
-  if (head_dim != kHeadDim || num_heads < 16 || num_heads > kMaxHeads || num_heads % 16 || num_tokens < 0 ||
-      num_tokens > 65535 || block_size < 1 || num_blocks < 1 || num_blocks > (int64_t(1) << 31) - 1 ||
+  if (next_n < 1 || next_n > 65535 || num_requests < 0 || num_requests > 65535) return GLM53_ERR_BAD_SHAPE;
+  const int64_t num_tokens = num_requests * next_n;
+  if (head_dim != kHeadDim || num_heads < 16 || num_heads > kMaxHeads || num_heads % 16 || num_tokens > 65535 || block_size < 1 || num_blocks < 1 || num_blocks > (int64_t(1) << 31) - 1 ||
       max_blocks < 1 || max_len < 0 || max_len > (int64_t(1) << 30) ||
       max_blocks * block_size > (int64_t(1) << 31) - 1 || page_bytes < block_size * (kHeadDim + 4) ||
       sq_h < kHeadDim || sq_t < num_heads * sq_h || sw_t < num_heads || sl_t < max_len ||
@@ -1263,7 +1336,7 @@ extern "C" int glm53_fp8_paged_mqa_logits(const void* q, int64_t sq_t, int64_t s
   // rows (one resident round at 2 workgroups per CU), 1 to 16 groups; one
   // group when groups straddle pages (block_size % 16 != 0).
   const bool al = block_size % 16 == 0;
-  if (bt_stride == 0 && al && num_tokens >= 16) {
+  if (bt_stride == 0 && al && next_n == 1 && num_tokens >= 16) {
     // one table shared by every row (a request's prefill chunk): 16 rows x
     // kRowsRun keys per workgroup, shorter runs while they leave fewer than
     // 1024 workgroups (four per CU; a workgroup loads its 16 rows' queries
@@ -1271,7 +1344,7 @@ extern "C" int glm53_fp8_paged_mqa_logits(const void* q, int64_t sq_t, int64_t s
     LogitsArgs a{static_cast<const uint8_t*>(q), sq_t, sq_h, static_cast<const uint8_t*>(kv_cache), page_bytes,
                  static_cast<int>(block_size), static_cast<int>(num_blocks), weights, sw_t, context_lens,
                  block_table, 0, static_cast<int>(max_blocks), static_cast<int>(num_heads),
-                 static_cast<int>(max_len), kRowsRun, logits, sl_t, clean_logits ? 1 : 0};
+                 static_cast<int>(max_len), kRowsRun, logits, sl_t, clean_logits ? 1 : 0, 1, 1};
     const int64_t row_blocks = (num_tokens + 4 * kLogitWaves - 1) / (4 * kLogitWaves);
     while (a.keys_per_wg > 128 && row_blocks * ((max_len + a.keys_per_wg - 1) / a.keys_per_wg) < 1024) a.keys_per_wg /= 2;
     const dim3 grid(static_cast<unsigned>((max_len + a.keys_per_wg - 1) / a.keys_per_wg), static_cast<unsigned>(row_blocks));
@@ -1287,18 +1360,22 @@ extern "C" int glm53_fp8_paged_mqa_logits(const void* q, int64_t sq_t, int64_t s
                        static_cast<int>(num_tokens));
     return static_cast<int>(hipGetLastError());
   }
-  const int64_t groups = num_tokens * ((max_len + 15) / 16);
+  const int tiles = static_cast<int>(num_heads / 16);
+  const int rows = rows_per_wg(next_n, tiles, al, num_requests * ((max_len + 15) / 16));
+  const int64_t row_blocks = (next_n + rows - 1) / rows;
+  const int64_t groups = num_requests * row_blocks * ((max_len + 15) / 16);
   int gpw = 1;
   while (al && gpw < 16 && groups >= int64_t(kLogitWaves) * 512 * gpw * 2) gpw *= 2;
   const int keys_per_wg = 16 * kLogitWaves * gpw;
   LogitsArgs a{static_cast<const uint8_t*>(q), sq_t, sq_h, static_cast<const uint8_t*>(kv_cache), page_bytes,
                static_cast<int>(block_size), static_cast<int>(num_blocks), weights, sw_t, context_lens,
                block_table, bt_stride, static_cast<int>(max_blocks), static_cast<int>(num_heads),
-               static_cast<int>(max_len), keys_per_wg, logits, sl_t, clean_logits ? 1 : 0};
-  const dim3 grid(static_cast<unsigned>((max_len + keys_per_wg - 1) / keys_per_wg), static_cast<unsigned>(num_tokens));
+               static_cast<int>(max_len), keys_per_wg, logits, sl_t, clean_logits ? 1 : 0, static_cast<int>(next_n),
+               static_cast<int>(row_blocks)};
+  const dim3 grid(static_cast<unsigned>((max_len + keys_per_wg - 1) / keys_per_wg),
+                  static_cast<unsigned>(num_requests * row_blocks));
   (void)hipGetLastError();
-  const int tiles = static_cast<int>(num_heads / 16);
-  LogitsKernel kernel = al ? pick_logits_kernel<true>(tiles, gpw) : pick_logits_kernel<false>(tiles, 1);
+  LogitsKernel kernel = pick_logits_kernel(tiles, gpw, rows, next_n > 1, al);
   hipLaunchKernelGGL(kernel, grid, dim3(kLogitThreads), 0, static_cast<hipStream_t>(stream), a.ctx, a.bt,
                      a.bt_stride, a.q, a.sq_t, a.keys_per_wg, a.max_len, a.block_size, a.max_blocks, a);
   return static_cast<int>(hipGetLastError());
@@ -1389,10 +1466,10 @@ bool topk_shape_ok(int64_t num_rows, int64_t max_len, int64_t k) {
 template <int P>
 void launch_final(bool cand, dim3 grid, hipStream_t st, const TopkArgs& a) {
   // the fields of the first loads lead as scalar arguments (preloaded into SGPRs)
-  void (*kernel)(const int32_t*, int, int, int, uint32_t*, int32_t*, int32_t*, int64_t, int, TopkArgs) =
+  void (*kernel)(const int32_t*, int, int, int, uint32_t*, int32_t*, int32_t*, int64_t, int, int, TopkArgs) =
       cand ? topk_final_kernel<P, true> : topk_final_kernel<P, false>;
   hipLaunchKernelGGL(kernel, grid, dim3(kFinalThreads), 0, st, a.lengths, a.max_len, a.k, a.chunks, a.cand_key,
-                     a.cand_pos, a.out, a.so, a.chunk_len, a);
+                     a.cand_pos, a.out, a.so, a.chunk_len, a.next_n, a);
 }
 
 }  // namespace
@@ -1412,15 +1489,22 @@ extern "C" int64_t glm53_indexer_topk_workspace_bytes(int64_t num_rows, int64_t 
 extern "C" int glm53_indexer_topk(const float* logits, int64_t sl, const int32_t* lengths, int64_t num_rows,
                                   int64_t max_len, int64_t k, void* workspace, int64_t workspace_bytes,
                                   int32_t* out, int64_t so, void* stream) {
+  return glm53_indexer_topk_next_n(logits, sl, lengths, num_rows, 1, max_len, k, workspace, workspace_bytes, out, so,
+                                   stream);
+}
+
+extern "C" int glm53_indexer_topk_next_n(const float* logits, int64_t sl, const int32_t* lengths, int64_t num_rows,
+                                         int64_t next_n, int64_t max_len, int64_t k, void* workspace,
+                                         int64_t workspace_bytes, int32_t* out, int64_t so, void* stream) {
   if (!logits || !lengths || !out) return GLM53_ERR_NULL_POINTER;
-  if (!topk_shape_ok(num_rows, max_len, k) || sl < max_len || so < k) return GLM53_ERR_BAD_SHAPE;
+  if (next_n < 1 || next_n > (int64_t(1) << 30) || num_rows % next_n || !topk_shape_ok(num_rows, max_len, k) || sl < max_len || so < k) return GLM53_ERR_BAD_SHAPE;
   if (num_rows == 0) return 0;
   if (!aligned(logits, 4)) return GLM53_ERR_MISALIGNED;
   const TopkPlan plan = plan_topk(num_rows, max_len, k);
   const int64_t need = topk_ws_bytes(plan, num_rows, k);
   if (need && (!workspace || workspace_bytes < need || !aligned(workspace, 16))) return GLM53_ERR_WORKSPACE;
   TopkArgs a{logits, sl, lengths, static_cast<int>(max_len), static_cast<int>(k), out, so, nullptr, nullptr,
-             plan.chunks, plan.chunk_len, aligned(logits, 16) && sl % 4 == 0};
+             plan.chunks, plan.chunk_len, aligned(logits, 16) && sl % 4 == 0, static_cast<int>(next_n)};
   if (need) {
     a.cand_key = static_cast<uint32_t*>(workspace);
     a.cand_pos = reinterpret_cast<int32_t*>(a.cand_key + num_rows * plan.chunks * k);
@@ -1431,7 +1515,7 @@ extern "C" int glm53_indexer_topk(const float* logits, int64_t sl, const int32_t
   if (row_plan(num_rows, max_len, k)) {
     const bool narrow = num_rows >= 256 && max_len <= 24576;
     hipLaunchKernelGGL((narrow ? topk_row_kernel<512> : topk_row_kernel<1024>), rows_grid, dim3(narrow ? 512 : 1024), 0,
-                       st, a.logits, a.sl, a.lengths, a.max_len, a.k, a.vec ? 1 : 0, a.out, a.so);
+                       st, a.logits, a.sl, a.lengths, a.max_len, a.k, a.vec ? 1 : 0, a.out, a.so, a.next_n);
     return static_cast<int>(hipGetLastError());
   }
   if (plan.mode == TopkPlan::kSweepMode) {
@@ -1442,7 +1526,7 @@ extern "C" int glm53_indexer_topk(const float* logits, int64_t sl, const int32_t
   if (cand) {
     const dim3 grid(static_cast<unsigned>(num_rows), static_cast<unsigned>(plan.chunks));
     // the fields of the first loads lead as scalar arguments (preloaded into SGPRs)
-#define CHUNK_LEAD a.logits, a.sl, a.lengths, a.max_len, a.k, a.chunk_len, a.chunks, a.vec ? 1 : 0, a
+#define CHUNK_LEAD a.logits, a.sl, a.lengths, a.max_len, a.k, a.chunk_len, a.chunks, a.vec ? 1 : 0, a.next_n, a
     if (plan.chunk_threads == kChunkThreadsWide)
       hipLaunchKernelGGL((topk_chunk_kernel<8, kChunkThreadsWide>), grid, dim3(kChunkThreadsWide), 0, st,
                          CHUNK_LEAD);

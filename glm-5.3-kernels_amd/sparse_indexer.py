@@ -62,20 +62,20 @@ def fp8_paged_mqa_logits(q: torch.Tensor, kv_cache: torch.Tensor, weights: torch
     qrows = qb.reshape(T, H, HEAD_DIM) if qb.is_contiguous() else qb.contiguous().reshape(T, H, HEAD_DIM)
     bt = block_tables if block_tables.stride(1) == 1 else block_tables.contiguous()
     ctx = context_lens.contiguous()
-    if next_n > 1:   # one row per query token: its own causal length, its request's block table
-        offs = torch.arange(next_n, device=ctx.device, dtype=torch.int32) - (next_n - 1)
-        ctx = (ctx[:, None] + offs[None, :]).reshape(T).contiguous()
-        bt = bt.repeat_interleave(next_n, dim=0).contiguous()
+    bt_stride = bt.stride(0)
+    if next_n > 1 and 0 < bt_stride < bt.shape[1]:   # rows that overlap (or, of one request, any stride)
+        bt = bt.clone(memory_format=torch.contiguous_format)
+        bt_stride = bt.shape[1]
     logits = torch.empty((T, max_model_len), dtype=torch.float32, device=q.device)
     if T == 0 or max_model_len == 0:
         return logits
     L = _lib.load()
     with torch.cuda.device(q.device):
-        rc = L.glm53_fp8_paged_mqa_logits(qrows.data_ptr(), qrows.stride(0), qrows.stride(1), kvb.data_ptr(),
-                                          kvb.stride(0), bs, nb, weights.data_ptr(), weights.stride(0),
-                                          ctx.data_ptr(), bt.data_ptr(), bt.stride(0), bt.shape[1], T, H,
-                                          HEAD_DIM, max_model_len, int(bool(clean_logits)), logits.data_ptr(),
-                                          logits.stride(0), _lib.stream_handle(q.device))
+        rc = L.glm53_fp8_paged_mqa_logits_next_n(qrows.data_ptr(), qrows.stride(0), qrows.stride(1), kvb.data_ptr(),
+                                                 kvb.stride(0), bs, nb, weights.data_ptr(), weights.stride(0),
+                                                 ctx.data_ptr(), bt.data_ptr(), bt_stride, bt.shape[1], B, next_n,
+                                                 H, HEAD_DIM, max_model_len, int(bool(clean_logits)),
+                                                 logits.data_ptr(), logits.stride(0), _lib.stream_handle(q.device))
     _lib.check(rc, "glm53_fp8_paged_mqa_logits")
     return logits
 
@@ -86,9 +86,15 @@ def indexer_topk(logits: torch.Tensor, lengths: torch.Tensor, k: int = 512) -> t
     fewer than k valid positions)."""
     if logits.dtype != torch.float32 or logits.dim() != 2 or logits.stride(1) != 1:
         raise ValueError("logits must be fp32 [rows, n] with contiguous rows")
-    rows, n = logits.shape
-    if lengths.dtype != torch.int32 or lengths.numel() != rows:
+    if lengths.dtype != torch.int32 or lengths.numel() != logits.shape[0]:
         raise ValueError("lengths must be int32 [rows]")
+    return _topk_rows(logits, lengths, 1, k)
+
+
+def _topk_rows(logits: torch.Tensor, lengths: torch.Tensor, next_n: int, k: int) -> torch.Tensor:
+    """indexer_topk of rows in groups of next_n: lengths int32 [rows / next_n],
+    those of each group's last row, the others one less each."""
+    rows, n = logits.shape
     if not 1 <= k <= n:
         raise ValueError(f"1 <= k <= {n} required, got {k}")
     out = torch.empty((rows, k), dtype=torch.int32, device=logits.device)
@@ -98,9 +104,9 @@ def indexer_topk(logits: torch.Tensor, lengths: torch.Tensor, k: int = 512) -> t
     ws_bytes = int(L.glm53_indexer_topk_workspace_bytes(rows, n, k))
     ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=logits.device)
     with torch.cuda.device(logits.device):
-        rc = L.glm53_indexer_topk(logits.data_ptr(), logits.stride(0), lengths.contiguous().data_ptr(), rows, n, k,
-                                  ws.data_ptr(), ws_bytes, out.data_ptr(), out.stride(0),
-                                  _lib.stream_handle(logits.device))
+        rc = L.glm53_indexer_topk_next_n(logits.data_ptr(), logits.stride(0), lengths.contiguous().data_ptr(), rows,
+                                         next_n, n, k, ws.data_ptr(), ws_bytes, out.data_ptr(), out.stride(0),
+                                         _lib.stream_handle(logits.device))
     _lib.check(rc, "glm53_indexer_topk")
     return out
 
@@ -117,10 +123,10 @@ def indexer_decode_pool_topk(q: torch.Tensor, kv_cache: torch.Tensor, weights: t
     B, next_n = q.shape[0], q.shape[1]
     lens = context_lens.to(torch.int32)
     cap = block_tables.shape[1] * kv_cache.shape[1]
-    if next_n == 1 and min(max_model_len, cap) >= k:
+    if next_n >= 1 and min(max_model_len, cap) >= k:
         # the top-k clamps each row's length to the columns it is given: the
         # columns the block table can hold (no separate clamp launch)
-        return indexer_topk(logits[:, :min(max_model_len, cap)], lens.contiguous(), k)
+        return _topk_rows(logits[:, :min(max_model_len, cap)], lens, next_n, k)
     if next_n > 1:
         offs = torch.arange(next_n, device=lens.device, dtype=torch.int32) - (next_n - 1)
         lens = (lens[:, None] + offs[None, :]).reshape(-1)

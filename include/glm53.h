@@ -368,6 +368,23 @@ int glm53_fp8_paged_mqa_logits(const void* q, int64_t sq_t, int64_t sq_h,
                                int64_t max_len, int clean_logits,
                                float* logits, int64_t sl_t, void* stream);
 
+/* The same for num_requests requests of next_n query rows each (a speculative
+ * step): rows are [num_requests * next_n], context_lens [num_requests] and
+ * block_table [num_requests][max_blocks]; row i of request b sees positions
+ * j < context_lens[b] - (next_n - 1) + i. */
+int glm53_fp8_paged_mqa_logits_next_n(const void* q, int64_t sq_t, int64_t sq_h,
+                                      const void* kv_cache, int64_t page_bytes,
+                                      int64_t block_size, int64_t num_blocks,
+                                      const float* weights, int64_t sw_t,
+                                      const int32_t* context_lens,
+                                      const int32_t* block_table,
+                                      int64_t bt_stride, int64_t max_blocks,
+                                      int64_t num_requests, int64_t next_n,
+                                      int64_t num_heads, int64_t head_dim,
+                                      int64_t max_len, int clean_logits,
+                                      float* logits, int64_t sl_t,
+                                      void* stream);
+
 /*
  * Top-k per row of the indexer logits: the top-512 pool selection whose pool
  * ids (topk_dst / pool_topk) the kpool expansion consumes
@@ -390,6 +407,14 @@ int glm53_indexer_topk(const float* logits, int64_t sl, const int32_t* lengths,
                        int64_t num_rows, int64_t max_len, int64_t k,
                        void* workspace, int64_t workspace_bytes,
                        int32_t* out, int64_t so, void* stream);
+
+/* The same for num_rows = requests * next_n rows: lengths [requests], and row i
+ * of request b has lengths[b] - (next_n - 1) + i valid columns. */
+int glm53_indexer_topk_next_n(const float* logits, int64_t sl,
+                              const int32_t* lengths, int64_t num_rows,
+                              int64_t next_n, int64_t max_len, int64_t k,
+                              void* workspace, int64_t workspace_bytes,
+                              int32_t* out, int64_t so, void* stream);
 
 /*
  * Diagnostic, no counterpart in the reference: stream `bytes` (a multiple of

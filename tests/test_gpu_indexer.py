@@ -498,3 +498,43 @@ def test_topk_filtered_rows(cuda, oracle, rows, n, k):
             sel = got[40 + r, :m]
             assert (np.diff(sel) > 0).all() and sel[-1] < ls[r] and (got[40 + r, m:] == -1).all()
             assert np.array_equal(np.sort(xs[r, sel]), np.sort(xs[r, :ls[r]])[-m:])
+
+
+@pytest.mark.parametrize("next_n", [2, 3, 4, 5, 9])
+@pytest.mark.parametrize("H", [16, 32, 48, 64])
+def test_next_n_rows_share_loads(cuda, next_n, H):
+    """The rows of a speculative step, scored two or four to a workgroup,
+    against the same rows as requests of their own (next_n = 1, expanded
+    lengths and tables): bit-identical logits and the same pools, for lengths
+    below next_n, negative, around a page's end and past the table, pages
+    outside the cache, pages that split 16-key groups, overlapping and shared
+    table rows, and every number of groups per wave."""
+    import torch
+    from sparse_indexer import fp8_paged_mqa_logits, indexer_decode_pool_topk, indexer_topk
+    g = W.gen(cuda, 5 * next_n + H)
+    for bs, per_req, max_len, k in ((64, 8, 512, 64), (64, 20, 1300, 512), (24, 30, 700, 700), (16, 200, 3200, 512),
+                                    (64, 100, 6400, 512), (64, 320, 20480, 512)):
+        lens = [0, 1, next_n - 1, -3, per_req * bs, per_req * bs + next_n, max_len // 2 + 1, 64 + next_n // 2]
+        B = len(lens)
+        q = (torch.randn(B, next_n, H, 128, generator=g, device=cuda) * 80).to(torch.float8_e4m3fn)
+        w = torch.randn(B * next_n, H, generator=g, device=cuda)
+        nb = B * per_req
+        cache = torch.randint(0, 120, (nb, bs, 1, 132), generator=g, device=cuda, dtype=torch.uint8)
+        cache.view(nb, -1)[:, bs * 128:] = (torch.rand(nb, bs, generator=g, device=cuda) - 0.2).view(torch.uint8)
+        ctx = torch.tensor(lens, device=cuda, dtype=torch.int32)
+        wide = torch.randint(0, nb, (B, per_req + 3), generator=g, device=cuda, dtype=torch.int32)
+        wide[4, 1], wide[5, per_req // 2] = -1, nb
+        tables = [wide[:, :per_req]]
+        if max_len == 1300:
+            tables += [wide[:1, :per_req].expand(B, per_req), wide.view(-1).as_strided((B, per_req), (3, 1))]
+        for bt in tables:
+            log_case("indexer logits next_n", next_n, H, bs, per_req, max_len, bt.stride(0))
+            rows_ctx = (ctx[:, None] + torch.arange(next_n, device=cuda, dtype=torch.int32) - (next_n - 1)).reshape(-1)
+            rows_bt = bt.repeat_interleave(next_n, 0).contiguous()
+            rows_q = q.view(B * next_n, 1, H, 128)
+            want = fp8_paged_mqa_logits(rows_q, cache, w, rows_ctx, rows_bt, max_len)
+            got = fp8_paged_mqa_logits(q, cache, w, ctx, bt, max_len)
+            assert torch.equal(got, want)
+            pools = indexer_decode_pool_topk(q, cache, w, ctx, bt, max_len, k=k)
+            cap = min(max_len, per_req * bs)
+            assert torch.equal(pools, indexer_topk(want[:, :cap], rows_ctx, min(k, cap)))
