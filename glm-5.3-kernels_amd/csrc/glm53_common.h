@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
+
 #include "glm53.h"
 
 namespace glm53 {
@@ -51,6 +53,19 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
   v = mx(a[0], a[1]);
   const auto b = __builtin_amdgcn_permlane32_swap(v, v, false, false);
   return mx(b[0], b[1]);
+}
+
+// Compute units of the current device (looked up once per device).
+inline int num_cus() {
+  static std::atomic<int> cached[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  int n = cached[dev].load(std::memory_order_relaxed);
+  if (!n) {
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1) n = 256;
+    cached[dev].store(n, std::memory_order_relaxed);
+  }
+  return n;
 }
 
 }  // namespace glm53

@@ -1284,6 +1284,25 @@ LogitsKernel pick_logits_rows(int gpw, int rows, bool spec, bool al) {
   return pick_logits_n<kTiles, 2, true>(gpw);
 }
 
+// Keys of a workgroup of fp8_mqa_logits_rows_kernel, a multiple of the 64 of a
+// chunk.  Two workgroups per compute unit already reach its rate (1.2 chunks a us;
+// one 0.87, three 1.1), so a call that fits the units so with runs of at most
+// eight chunks takes the shortest such run, in one round: 128 rows x 30000 keys, 32
+// heads 29.7 -> 24.3 us (128-key runs in 1880 workgroups before), 300 x 6000 18.3 ->
+// 16.1, 33 x 50000, 48 heads 27.1 -> 21.2, 250 x 12000, 64 heads 45.5 -> 33.8.  Larger
+// calls halve 1024 keys while that leaves fewer than four workgroups per unit: there
+// lengths between the powers of two are no better (1500 x 40000: 16 chunks 234 us,
+// 15 240, 13 246; 700 x 20000: 8 62.3, 11 64.0, 14 66).
+int rows_run(int64_t row_blocks, int64_t max_len) {
+  const int64_t cus = num_cus();
+  const auto workgroups = [&](int keys) { return row_blocks * ((max_len + keys - 1) / keys); };
+  for (int keys = 64; keys <= 512; keys += 64)
+    if (workgroups(keys) <= 2 * cus) return keys;
+  int keys = kRowsRun;
+  while (keys > 512 && workgroups(keys) < 4 * cus) keys /= 2;
+  return keys;
+}
+
 // Kernel for 16 * tiles heads and gpw groups per wave (unaligned block
 // sizes: one group per wave).
 LogitsKernel pick_logits_kernel(int tiles, int gpw, int rows, bool spec, bool al) {
@@ -1338,15 +1357,13 @@ extern "C" int glm53_fp8_paged_mqa_logits_next_n(const void* q, int64_t sq_t, in
   const bool al = block_size % 16 == 0;
   if (bt_stride == 0 && al && next_n == 1 && num_tokens >= 16) {
     // one table shared by every row (a request's prefill chunk): 16 rows x
-    // kRowsRun keys per workgroup, shorter runs while they leave fewer than
-    // 1024 workgroups (four per CU; a workgroup loads its 16 rows' queries
-    // once per run)
+    // rows_run keys per workgroup
     LogitsArgs a{static_cast<const uint8_t*>(q), sq_t, sq_h, static_cast<const uint8_t*>(kv_cache), page_bytes,
                  static_cast<int>(block_size), static_cast<int>(num_blocks), weights, sw_t, context_lens,
                  block_table, 0, static_cast<int>(max_blocks), static_cast<int>(num_heads),
-                 static_cast<int>(max_len), kRowsRun, logits, sl_t, clean_logits ? 1 : 0, 1, 1};
+                 static_cast<int>(max_len), 0, logits, sl_t, clean_logits ? 1 : 0, 1, 1};
     const int64_t row_blocks = (num_tokens + 4 * kLogitWaves - 1) / (4 * kLogitWaves);
-    while (a.keys_per_wg > 128 && row_blocks * ((max_len + a.keys_per_wg - 1) / a.keys_per_wg) < 1024) a.keys_per_wg /= 2;
+    a.keys_per_wg = rows_run(row_blocks, max_len);
     const dim3 grid(static_cast<unsigned>((max_len + a.keys_per_wg - 1) / a.keys_per_wg), static_cast<unsigned>(row_blocks));
     void (*kernel)(LogitsArgs, int);
     switch (num_heads / 16) {

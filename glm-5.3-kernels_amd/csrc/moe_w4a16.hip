@@ -745,19 +745,6 @@ extern "C" int glm53_moe_w4a16_repack(const void* w_packed, const void* w_scale,
 
 namespace {
 
-// Compute units of the current device (cached per device).
-int num_cus() {
-  static int cached[64] = {0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (!cached[dev]) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1) n = 256;
-    cached[dev] = n;
-  }
-  return cached[dev];
-}
-
 int launch_gate_up(bool self_align, const void* x, int64_t sx, const void* w13, const void* s13,
                    const int32_t* sorted_ids, const int32_t* expert_ids, const void* topk_ids, int ids_is_i64,
                    int64_t num_routes, int64_t topk, int64_t num_experts, int64_t n_inter, int64_t hidden,

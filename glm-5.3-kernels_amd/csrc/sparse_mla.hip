@@ -46,7 +46,6 @@
 //     same way); see sparse_mla_kernel.
 #include "glm53_common.h"
 
-#include <atomic>
 
 namespace glm53 {
 namespace {
@@ -1645,19 +1644,6 @@ int64_t tokens_grid(int64_t num_tokens, int heads_padded, int64_t num_splits) {
   if (heads_padded != kHeads || num_tokens < 3 || num_tokens > 7 || num_tokens == 4) return num_tokens;
   const int64_t tp = num_tokens == 3 ? 4 : 8;
   return num_splits <= 32 * (8 / tp) ? tp : num_tokens;   // each XCD's share within its 32 CUs
-}
-
-// Compute units of the current device (looked up once per device).
-int num_cus() {
-  static std::atomic<int> cached[64];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  int n = cached[dev].load(std::memory_order_relaxed);
-  if (!n) {
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1) n = 256;
-    cached[dev].store(n, std::memory_order_relaxed);
-  }
-  return n;
 }
 
 // Multiplier of fast_div: n / d = mulhi(n, mul) >> sh for 0 <= n < 2^31.  With

@@ -427,6 +427,31 @@ def test_shared_table_rows_kernel(cuda, oracle, heads):
         check_logits(oracle, got, q, cache, w, lens, shared.contiguous(), pools, clean, rows=range(0, T, 6))
 
 
+@pytest.mark.parametrize("heads,bs,pools,T", [(32, 64, 1000, 16), (32, 64, 9000, 128), (48, 16, 50001, 33),
+                                              (64, 64, 12000, 250), (32, 48, 15999, 200), (16, 64, 9000, 400)])
+def test_rows_kernel_run_lengths(cuda, heads, bs, pools, T):
+    """Runs of 1, 3, 5, 6, 7 and 8 chunks of 64 keys per workgroup (the lengths
+    that fit two workgroups per compute unit), the last run ragged:
+    bit-identical to the per-token kernel, rows of their own lengths."""
+    import torch
+    from sparse_indexer import fp8_paged_mqa_logits
+    g = torch.Generator(device=cuda).manual_seed(heads + pools + T)
+    cache, nb = W.indexer_cache(cuda, g, pools + bs, bs)
+    per_req = (pools + bs - 1) // bs
+    table = torch.randperm(nb, generator=g, device=cuda).to(torch.int32)[:per_req]
+    lens = torch.randint(0, pools + 1, (T,), generator=g, device=cuda, dtype=torch.int32)
+    lens[:2] = torch.tensor([pools, pools - 1], dtype=torch.int32, device=cuda)
+    qf = torch.randn(T, 1, heads, 128, generator=g, device=cuda)
+    q = (qf * (448.0 / qf.abs().amax(dim=-1, keepdim=True))).to(torch.float8_e4m3fn)
+    w = (torch.randn(T, heads, generator=g, device=cuda) * heads ** -0.5).contiguous()
+    shared = table[None, :].expand(T, per_req)
+    log_case("indexer run lengths", heads, bs, pools, T)
+    got = fp8_paged_mqa_logits(q, cache, w, lens, shared, pools)
+    ref = fp8_paged_mqa_logits(q, cache, w, lens, shared.contiguous(), pools)
+    torch.cuda.synchronize()
+    assert torch.equal(got, ref)
+
+
 @pytest.mark.parametrize("heads,bs,pools,T", [(16, 16, 1023, 16), (48, 48, 1025, 33), (32, 64, 64, 17),
                                               (64, 128, 2049, 64), (32, 16, 15, 20)])
 def test_shared_table_run_edges(cuda, heads, bs, pools, T):
