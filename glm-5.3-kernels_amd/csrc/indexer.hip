@@ -867,8 +867,8 @@ __global__ __launch_bounds__(kThreads) void topk_chunk_kernel(
 // filled one: never selected.
 template <int P, bool kCand>
 __global__ __launch_bounds__(kFinalThreads) void topk_final_kernel(
-    const int32_t* p_lengths, int p_max_len, int p_k, int p_chunks, uint32_t* p_cand_key, int32_t* p_cand_pos,
-    int32_t* p_out, int64_t p_so, int p_chunk_len, int p_next_n, const TopkArgs a) {
+    const int32_t* p_lengths, int p_max_len, int p_k, int p_chunks, int p_next_n, uint32_t* p_cand_key,
+    int32_t* p_cand_pos, int32_t* p_out, int64_t p_so, int p_chunk_len, const TopkArgs a) {
   __shared__ SelShared<kFinalThreads> sh;
   const int row = blockIdx.x, tid = threadIdx.x;
   const int len = clamp_len(p_lengths, p_max_len, row, p_next_n);
@@ -1006,8 +1006,8 @@ __device__ __forceinline__ float key_value(uint32_t key) {   // inverse of order
 
 template <int kThreads>
 __global__ __launch_bounds__(kThreads) void topk_row_kernel(
-    const float* p_logits, int64_t p_sl, const int32_t* p_lengths, int p_max_len, int p_k, int p_vec,
-    int32_t* p_out, int64_t p_so, int p_next_n) {
+    const float* p_logits, int64_t p_sl, const int32_t* p_lengths, int p_max_len, int p_k, int p_vec, int p_next_n,
+    int32_t* p_out, int64_t p_so) {
   constexpr int P = kListKeys / kThreads;      // list keys per thread
   constexpr int kRuns = P / 4;                 // sampled runs of 4 per thread
   constexpr int kVecs = 4;                     // 4-key loads per thread and step of the pass over the row
@@ -1482,11 +1482,12 @@ bool topk_shape_ok(int64_t num_rows, int64_t max_len, int64_t k) {
 
 template <int P>
 void launch_final(bool cand, dim3 grid, hipStream_t st, const TopkArgs& a) {
-  // the fields of the first loads lead as scalar arguments (preloaded into SGPRs)
-  void (*kernel)(const int32_t*, int, int, int, uint32_t*, int32_t*, int32_t*, int64_t, int, int, TopkArgs) =
+  // the fields of the first loads lead as scalar arguments (preloaded into
+  // SGPRs); next_n, which the length's address needs, among the first 14 dwords
+  void (*kernel)(const int32_t*, int, int, int, int, uint32_t*, int32_t*, int32_t*, int64_t, int, TopkArgs) =
       cand ? topk_final_kernel<P, true> : topk_final_kernel<P, false>;
-  hipLaunchKernelGGL(kernel, grid, dim3(kFinalThreads), 0, st, a.lengths, a.max_len, a.k, a.chunks, a.cand_key,
-                     a.cand_pos, a.out, a.so, a.chunk_len, a.next_n, a);
+  hipLaunchKernelGGL(kernel, grid, dim3(kFinalThreads), 0, st, a.lengths, a.max_len, a.k, a.chunks, a.next_n,
+                     a.cand_key, a.cand_pos, a.out, a.so, a.chunk_len, a);
 }
 
 }  // namespace
@@ -1532,7 +1533,7 @@ extern "C" int glm53_indexer_topk_next_n(const float* logits, int64_t sl, const 
   if (row_plan(num_rows, max_len, k)) {
     const bool narrow = num_rows >= 256 && max_len <= 24576;
     hipLaunchKernelGGL((narrow ? topk_row_kernel<512> : topk_row_kernel<1024>), rows_grid, dim3(narrow ? 512 : 1024), 0,
-                       st, a.logits, a.sl, a.lengths, a.max_len, a.k, a.vec ? 1 : 0, a.out, a.so, a.next_n);
+                       st, a.logits, a.sl, a.lengths, a.max_len, a.k, a.vec ? 1 : 0, a.next_n, a.out, a.so);
     return static_cast<int>(hipGetLastError());
   }
   if (plan.mode == TopkPlan::kSweepMode) {
