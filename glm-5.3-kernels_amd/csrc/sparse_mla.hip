@@ -46,7 +46,6 @@
 //     same way); see sparse_mla_kernel.
 #include "glm53_common.h"
 
-
 namespace glm53 {
 namespace {
 
