@@ -1013,7 +1013,11 @@ __global__ __launch_bounds__(kThreads) void topk_row_kernel(
   constexpr int kVecs = 4;                     // 4-key loads per thread and step of the pass over the row
   __shared__ SelShared<kThreads> sh;
   __shared__ int32_t list[kListKeys];
-  __shared__ uint32_t listed;
+  // Counters.  `listed` is read by every thread after list_keys' last barrier
+  // and set to 0 again only behind another one (those of radix_threshold); the
+  // ties have a counter of their own, since no barrier lies between that read
+  // and their first count.
+  __shared__ uint32_t listed, tied;
   const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
   const int len = clamp_len(p_lengths, p_max_len, row, p_next_n);
   const int k = p_k;
@@ -1133,7 +1137,7 @@ __global__ __launch_bounds__(kThreads) void topk_row_kernel(
     float f[P];
     load_sample(f);
     clear_hist(sh);
-    if (tid == 0) listed = 0;
+    if (tid == 0) listed = tied = 0;
     sample_keys(f, kmin, kmax);
     // one pass: the bin the rank falls in, whole
     const Threshold t = radix_threshold<kThreads, 1>(sh, [&](auto f) { for_each_key(kk, f); }, rank, kmin, kmax);
@@ -1147,7 +1151,7 @@ __global__ __launch_bounds__(kThreads) void topk_row_kernel(
     clear_hist(sh);
     sample_keys(f, kmin, kmax);
     const Threshold t = radix_threshold(sh, [&](auto f) { for_each_key(kk, f); }, rank, kmin, kmax);
-    if (tid == 0) listed = 0;
+    if (tid == 0) listed = 0;   // the first count was read before radix_threshold's barriers
     __syncthreads();
     n_list = list_keys([&](float v) { return order_key(v) > t.thr; });
     if (n_list < k) ties = t.thr;
@@ -1159,7 +1163,6 @@ __global__ __launch_bounds__(kThreads) void topk_row_kernel(
     // The list holds every key above `ties`: the first k - n_list positions
     // of that key complete it, collected step by step from the row's start.
     for (int i = tid; i < words; i += kThreads) gt[i] = eq[i] = 0u;
-    if (tid == 0) listed = 0;
     __syncthreads();
     for (int i = tid; i < n_list; i += kThreads) atomicOr(&gt[list[i] >> 5], 1u << (list[i] & 31));
     int found = 0;
@@ -1168,7 +1171,7 @@ __global__ __launch_bounds__(kThreads) void topk_row_kernel(
       load_step(base, cur);
       uint32_t hits = hits_of(cur, [&](float v) { return order_key(v) == ties; });
       const uint32_t n = wave_incl_scan(__popc(hits));
-      if (lane == 63 && n) atomicAdd(&listed, n);
+      if (lane == 63 && n) atomicAdd(&tied, n);
       while (hits) {
         const int b = __builtin_ctz(hits);
         hits &= hits - 1;
@@ -1176,8 +1179,8 @@ __global__ __launch_bounds__(kThreads) void topk_row_kernel(
         if (p < len) atomicOr(&eq[p >> 5], 1u << (p & 31));   // a NaN key (0) also stands past the row's end
       }
       __syncthreads();
-      found = static_cast<int>(listed);
-      __syncthreads();
+      found = static_cast<int>(tied);
+      __syncthreads();   // before the next step's counts
     }
     if (found < k - n_list) ties = ~0u;   // uniform
   }

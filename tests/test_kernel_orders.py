@@ -1,0 +1,76 @@
+"""Kernels of csrc/indexer.hip run on the host, in orders of their waves and
+lanes that a GPU takes rarely: the results must not depend on them."""
+import ctypes
+
+import numpy as np
+import pytest
+
+import host_kernels
+
+I64, P = ctypes.c_int64, ctypes.c_void_p
+ORDERS = [(0, 0), (0, 1), (1, 0), (1, 1)]   # waves, lanes: ascending or descending
+
+
+@pytest.fixture(scope="module")
+def lib(tmp_path_factory):
+    return host_kernels.build("indexer.hip", tmp_path_factory.mktemp("indexer"))
+
+
+def topk(lib, x, lens, k, max_len):
+    ws = lib.glm53_indexer_topk_workspace_bytes
+    ws.restype, ws.argtypes = I64, [I64, I64, I64]
+    run = lib.glm53_indexer_topk
+    run.argtypes = [P, I64, P, I64, I64, I64, P, I64, P, I64, P]
+    rows = x.shape[0]
+    out = np.full((rows, k + 2 * max_len), -7, np.int32)     # room past each row: a stray rank shows
+    need = ws(rows, max_len, k)
+    scratch = np.zeros(need + 64, np.uint8)
+    at = (scratch.ctypes.data + 63) // 64 * 64
+    assert run(x.ctypes.data, x.shape[1], lens.ctypes.data, rows, max_len, k, at, need, out.ctypes.data,
+               out.shape[1], None) == 0
+    assert (out[:, k:] == -7).all()
+    return out[:, :k]
+
+
+def rows_of(n, k):
+    """Rows that take every way through the selection: values that differ, a
+    tie that holds most of a row with fewer than k keys above it (zeros, -inf
+    or NaN), with more above it, few values, one value."""
+    rng = np.random.default_rng(n + k)
+    x = rng.standard_normal((8, n)).astype(np.float32)
+    few = np.zeros(n, bool)
+    few[::max(53, 2 * n // k)] = True
+    x[1] = np.where(few, np.abs(x[1]), 0)
+    x[2] = np.where(few, x[2], -np.inf)
+    x[3] = np.where(few, x[3], np.nan)
+    x[4] = np.where(rng.random(n) < 0.5, x[4], 0)
+    x[5] = rng.integers(0, 3, n)
+    x[6] = -1.5
+    x[7] = np.arange(n)
+    return x
+
+
+# the one-workgroup selection (4097..131072 columns, k <= 1024) at 1024 threads, its row as one list, its edges
+@pytest.mark.parametrize("n,k", [(4097, 512), (5001, 1024), (12001, 40), (16384, 512), (4000, 700)])
+@pytest.mark.parametrize("order", ORDERS)
+def test_topk_any_order(lib, oracle, n, k, order):
+    lib.host_hip_order(*order)
+    x = rows_of(n, k)
+    lens = np.array([n, n, n - 1, n, n - 3, n, n, k], np.int32)
+    assert np.array_equal(topk(lib, x, lens, k, n), oracle.indexer_topk(x, lens, k))
+
+
+@pytest.mark.parametrize("order", ORDERS)
+def test_topk_any_order_other_plans(lib, oracle, order):
+    """512-thread workgroups (256 rows), the two stages (few rows of 20000
+    columns) and the sweeps (more candidates than the final stage takes)."""
+    lib.host_hip_order(*order)
+    x = np.zeros((256, 5001), np.float32)
+    x[:8] = rows_of(5001, 512)
+    lens = np.zeros(256, np.int32)
+    lens[:8] = 5001
+    assert np.array_equal(topk(lib, x, lens, 512, 5001), oracle.indexer_topk(x, lens, 512))
+    for n, k in ((20000, 512), (34000, 20000)):
+        x = rows_of(n, k)[1:4]
+        lens = np.array([n, n - 5, n], np.int32)
+        assert np.array_equal(topk(lib, x, lens, k, n), oracle.indexer_topk(x, lens, k)), (n, k)
