@@ -38,9 +38,11 @@
 //     row-major in LDS and reads it back with ds_read_b64_tr_b16 (two reads
 //     per 16x32 operand).  O^T accumulates in 8 MFMA tiles per wave.
 //   * Splits longer than one chunk (batches of more than about 30 tokens, the
-//     prefill-shaped call's single split of 2176 keys per token) run
-//     sparse_mla_rows_kernel instead: every wave of a workgroup takes 16 whole
-//     rows of a unit of 64 or 128 keys, then a slice of the output.
+//     prefill-shaped call's single split of 2176 keys per token) run one of two
+//     other kernels, by the workgroups there are (rows_waves):
+//     sparse_mla_rows_kernel, where every wave of a workgroup takes 16 whole
+//     rows of a unit of 64 or 128 keys, then a slice of the output, and
+//     sparse_mla_pair_kernel, two waves per workgroup, a latent half each.
 //   * Workgroups are numbered so that a token's splits share an XCD (its L2
 //     holds the token's q and indices, and the merge kernel is numbered the
 //     same way); see sparse_mla_kernel.
@@ -1657,31 +1659,44 @@ Div div_magic(int64_t d) {
 }
 
 // Waves per workgroup of sparse_mla_rows_kernel for a long split, or 0 for
-// the pair kernel.  A compute unit holds one workgroup of 8 waves or two of 4
-// (a round of the former takes 51-57 us at 2176 keys, of the latter 62-66 with
-// one per CU and 90-107 with two): 8 waves where they need one round, or three
-// against the 4-wave form's half-filled second (640 workgroups 154 us against
-// 158, 700 156 / 163), but not for a few units (splits of 436 and 544 keys: 23.8
-// / 22.4 and 27.0 / 25.9 us at 48 and 64 tokens).  From three to three and a
-// half rounds the pair kernel, four workgroups to a CU, is still ahead (800:
-// 174 us against 183; 900: 189 / 188).  Row offsets are 32-bit counts of 16
-// bytes here; a flat cache that spans more keeps the pair kernel's 64 bits.
-int rows_waves(const MlaArgs& a, int mode, int64_t workgroups) {
+// the pair kernel.  A compute unit holds one workgroup of the rows kernel's 8
+// waves, two of its 4, or four of the pair kernel's 2.  Pair / rows, us, 512 and
+// 2176 indices (medians; flat caches of 262144 rows, half of a token's indices
+// within 4096 rows; 16 heads unless said):
+//   up to two per unit the rows kernel: 128 workgroups 40.6 / 21.3 and 80.1 /
+//     41.0, 256 31.1 / 24.3 and 106 / 61.2, 512 42.6 / 35.7 and 151 / 108;
+//     its 8 waves where they need one round, but not for short splits
+//     (436 and 544 keys: 23.8 / 22.4 and 27.0 / 25.9 us at 48 and 64 tokens);
+//   up to four the pair kernel, in one round: 513 43.3 / 53.8 and 151 / 156,
+//     768 46.8 / 61.1 and 167 / 171, 1024 (64 heads) 51.9 / 59.1 and 185 / 202;
+//   up to six the rows kernel, whose third round the pair kernel's second half
+//     fills: 1100 79.5 / 75.6 and 291 / 253, 1536 94.1 / 88.6 and 352 / 299;
+//   up to eight the pair kernel again: 1888 as 1 : 1.04 and 1 : 1.00, from a
+//     cache of 16384 rows 1 : 1.07 and 1 : 1.02, 64 heads 1 : 1.09 and 1 : 1.06;
+//   from eight on the gathers decide.  The pair kernel costs less per
+//     workgroup (16384 rows, 512 indices: 4096 workgroups 190 / 204, 6000 268 /
+//     294; 2176: 695 / 700 and 990 / 1012), the rows kernel less per gathered
+//     key: ahead with long splits of many tokens (2048 429 / 398, 4096 813 /
+//     776), not where head groups find the rows in L2 (512 tokens of 64
+//     heads 394 / 403).
+// Row offsets are 32-bit counts of 16 bytes there; a flat cache that spans
+// more keeps the pair kernel's 64 bits.
+int rows_waves(const MlaArgs& a, int mode, int64_t num_tokens, int64_t workgroups) {
   if (mode == kFlatRows && (a.skv < 0 || (a.seq_kv - 1) > int64_t(0xffffffff) / (a.skv / 16 > 0 ? a.skv / 16 : 1)))
     return 0;
   const int64_t cus = num_cus();
   if (workgroups <= cus) return a.split_len >= 640 ? 8 : 4;
   if (workgroups <= 2 * cus) return 4;
-  if (workgroups <= 3 * cus) return 8;
-  if (2 * workgroups <= 7 * cus) return 0;
-  return 4;
+  if (workgroups <= 4 * cus) return 0;
+  if (workgroups <= 6 * cus) return 4;
+  return workgroups >= 8 * cus && num_tokens >= 4 * cus && a.split_len >= 2048 ? 4 : 0;
 }
 
 void launch_attention(const MlaArgs& a, int64_t num_tokens, hipStream_t st) {
   // Splits longer than one chunk of gathers pipeline their chunks.
   const bool pipe = a.split_len > kChunkTiles * kTile;
-  // Long splits go to the pair kernel, whose masked keys read row 0 (page 0):
-  // it needs a non-empty cache (seq_kv counts rows, or pages when paged).
+  // Long splits go to the rows or the pair kernel, whose masked keys read row 0
+  // (page 0): they need a non-empty cache (seq_kv counts rows, or pages when paged).
   const bool pair = pipe && a.seq_kv > 0;
   // Splits of exactly three tiles (65 to 96 keys) run in one round on three
   // key groups, splits of one tile on one key group.
@@ -1712,7 +1727,7 @@ void launch_attention(const MlaArgs& a, int64_t num_tokens, hipStream_t st) {
       hipLaunchKernelGGL((sparse_mla_kernel<M, false, G>), grid, dim3(SplitShape<G>::kThreads), 0, st,       \
                          GLM53_LEAD);                                                                  \
   } while (0)
-  if (const int waves = pair ? rows_waves(a, mode, static_cast<int64_t>(grid.x) * grid.y * grid.z) : 0) {
+  if (const int waves = pair ? rows_waves(a, mode, num_tokens, static_cast<int64_t>(grid.x) * grid.y * grid.z) : 0) {
     MlaArgs ra = a;
     if (mode == kFlatRows) ra.row_units = static_cast<int>(static_cast<uint32_t>(a.skv / 16));
     const Div bd = div_magic(a.block_size), pd = div_magic(a.pool_size);

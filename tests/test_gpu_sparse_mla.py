@@ -39,7 +39,7 @@ def u16(t):
 
 def kernel_groups(topk, splits):
     """Online-softmax streams per split in the HIP kernel for this split
-    length: one past a chunk of 256 keys (the pair kernel) and for splits of
+    length: one past a chunk of 256 keys (the long-split kernels) and for splits of
     one 32-key tile (one key group), three key groups for splits of exactly
     three tiles, two otherwise."""
     split_len = -(-topk // splits)
@@ -578,8 +578,9 @@ def test_three_key_group_splits(cuda, oracle, small_cache):
 
 
 def test_long_split_pair_kernel_edges(cuda, oracle, small_cache):
-    """Splits longer than one chunk (256 indices) run on the pair kernel (one
-    online-softmax stream per split): against the reference's single stream
+    """Splits longer than one chunk (256 indices) in small batches (one
+    online-softmax stream per split; a handful of workgroups takes the rows
+    kernel, test_long_split_by_workgroups has the pair kernel's range): against the reference's single stream
     (groups=1, BLOCK_N=32) with odd tile counts (352 = 11 tiles, 288 = 9), a
     last split shorter than the others (1088 in 3 splits), split partials
     merged (2176 in 2 splits, 20 heads: a padded head group), pads and
@@ -612,8 +613,8 @@ def test_long_split_pair_kernel_edges(cuda, oracle, small_cache):
 
 @pytest.mark.parametrize("T,H,topk,splits", [
     (3, 16, 288, 1), (2, 20, 320, 1), (48, 16, 2176, 5), (12, 80, 2176, 8), (28, 80, 2176, 8),   # 64-key units
-    (2, 16, 640, 1), (3, 8, 672, 1), (5, 32, 2176, 2), (20, 80, 2176, 6),                         # 128-key units
-    (20, 80, 2176, 8)])                                                                           # the pair kernel
+    (2, 16, 640, 1), (3, 8, 672, 1), (5, 32, 2176, 2),                                            # 128-key units
+    (20, 80, 2176, 6), (20, 80, 2176, 8)])                                                        # the pair kernel
 def test_long_split_rows_kernel_edges(cuda, oracle, small_cache, T, H, topk, splits):
     """Splits of more than 256 keys in units of 64 or 128 keys: the last unit
     whole, half or a few keys, the first half of a row's indices masked (whole
@@ -643,6 +644,58 @@ def test_long_split_rows_kernel_edges(cuda, oracle, small_cache, T, H, topk, spl
     paged = triton_mla_sparse_attention_paged(q, pages, idx, req, table, W.SM_SCALE, num_kv_splits=splits)
     torch.cuda.synchronize()
     assert torch.equal(paged, out)
+
+
+# (workgroups per compute unit, workgroups more) -> tokens of one split or of five: each step of the kernel
+# choice from both sides, the pair kernel between 2 and 4 (and 6 and 8) per unit
+@pytest.mark.parametrize("per_cu,more,H,topk,splits", [
+    (2, 0, 16, 320, 1), (2, 1, 16, 288, 1), (3, 0, 8, 352, 1), (4, 0, 16, 2176, 1), (4, 1, 16, 288, 1),
+    (3, 2, 20, 1088, 1), (3, 0, 16, 2176, 5), (6, 0, 16, 352, 1), (6, 1, 16, 352, 1), (8, 0, 16, 2048, 1),
+    (8, -1, 16, 2048, 1)])
+def test_long_split_by_workgroups(cuda, oracle, small_cache, per_cu, more, H, topk, splits):
+    """Splits of more than 256 keys at the numbers of workgroups where the
+    kernel changes, flat, paged and pooled: odd tile counts (288 = 9 tiles,
+    352 = 11), a last split shorter than the others (2176 in 5), one split
+    straight to the output, padded head groups (8 and 20 heads), indices
+    outside the cache both ways, rows with only masked keys.  Some tokens
+    against the oracle, the paged form bit-identical, the pooled one to its
+    expansion."""
+    from sparse_utils import expand_pools_and_append_tail
+    from titan_mla import (triton_mla_sparse_attention, triton_mla_sparse_attention_paged,
+                           triton_mla_sparse_attention_pooled)
+    w, rows = small_cache
+    n = w["n_rows"]
+    kv = w["cache"].view(n, 1, 528)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    T = (per_cu * cus + more) // splits // -(-H // 16)
+    g = W.gen(cuda, 3000 + topk + T)
+    q = torch.randn(T, H, 512, generator=g, device=cuda).to(torch.bfloat16)
+    idx = torch.randint(-40, n + 40, (T, 1, topk), generator=g, device=cuda, dtype=torch.int32)
+    idx[0, :, topk // 2:] = -1
+    idx[T - 1, :, :topk // 2] = -1
+    idx[1] = -1
+    log_case("mla long splits by workgroups", T, H, topk, splits)
+    out = triton_mla_sparse_attention(q, kv, idx, W.SM_SCALE, num_kv_splits=splits)
+    torch.cuda.synchronize()
+    assert torch.equal(out[1], torch.zeros_like(out[1]))
+    some = sorted({0, 1, 2, T // 2, T - 2, T - 1})
+    want = oracle.sparse_mla(u16(q[some]), rows, idx[some].cpu().numpy(), W.SM_SCALE, n_splits=splits, groups=1,
+                             block_n=32)
+    compare(out[some], want, ("long splits by workgroups", T, H, topk, splits))
+    pages = w["cache"].view(n // 64, 64, 528)
+    table = torch.arange(n // 64, device=cuda, dtype=torch.int32)[None, :]
+    req = torch.zeros(T, dtype=torch.int32, device=cuda)
+    paged = triton_mla_sparse_attention_paged(q, pages, idx, req, table, W.SM_SCALE, num_kv_splits=splits)
+    assert torch.equal(paged, out)
+    pools = torch.randint(-2, n // 4 + 5, (T, topk // 4 - 1), generator=g, device=cuda, dtype=torch.int32)
+    seq = torch.randint(0, n, (T,), generator=g, device=cuda, dtype=torch.int32)
+    slots = torch.full((T, topk), -1, dtype=torch.int32, device=cuda)
+    slots[:, :topk - 1] = expand_pools_and_append_tail(pools, seq, 4)
+    fused = triton_mla_sparse_attention_pooled(q, pages, pools, seq, 4, req, table, W.SM_SCALE, topk=topk,
+                                               num_kv_splits=splits)
+    paged = triton_mla_sparse_attention_paged(q, pages, slots, req, table, W.SM_SCALE, num_kv_splits=splits)
+    torch.cuda.synchronize()
+    assert torch.equal(fused, paged)
 
 
 @pytest.mark.parametrize("topk", [288, 1088])
