@@ -42,6 +42,8 @@
 // top k), then one workgroup per row selects from those candidates.  Keys
 // stay in registers (thread-contiguous runs of positions) through every
 // pass; rows too long for the two stages are re-read from L2 per pass.
+#include <type_traits>
+
 #include "glm53_common.h"
 
 namespace glm53 {
@@ -643,10 +645,12 @@ struct Threshold {
 // bins, which keeps the histogram atomics from piling onto a few addresses.
 // for_keys(f) calls f(key) for every key of this thread; the keys matching
 // the shared bits must number at least k.  The caller has zeroed both
-// histograms (clear_hist) before the call.
-template <int kThreads, int kMaxPasses = 3, class ForKeys>
+// histograms (clear_hist) before the call.  With kCoarse the search also ends
+// at a bin whose keys and the ones above number at most `enough`, and *taken is
+// that number (at least k; ~0u when all keys are one).
+template <int kThreads, bool kCoarse = false, class ForKeys>
 __device__ Threshold radix_threshold(SelShared<kThreads>& sh, ForKeys for_keys, uint32_t k, uint32_t kmin,
-                                     uint32_t kmax) {
+                                     uint32_t kmax, uint32_t enough = 0, uint32_t* taken = nullptr) {
   constexpr int kWaves = kThreads / 64;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   kmin = ~wave_max(~kmin);
@@ -656,11 +660,14 @@ __device__ Threshold radix_threshold(SelShared<kThreads>& sh, ForKeys for_keys, 
 #pragma unroll
   for (int i = 0; i < kWaves; i++) { kmin = min(kmin, sh.wmin[i]); kmax = max(kmax, sh.wmax[i]); }
   const uint32_t diff = kmin ^ kmax;
-  if (diff == 0) return {kmax, ~0u, k};   // one distinct key
+  if (diff == 0) {   // one distinct key
+    if constexpr (kCoarse) *taken = ~0u;
+    return {kmax, ~0u, k};
+  }
   int top = 32 - __clz(static_cast<int>(diff));   // bits [top, 32) are shared
   uint32_t pmask = top == 32 ? 0u : ~((1u << top) - 1u);
   uint32_t prefix = kmax & pmask, need = k;
-  for (int pass = 0; top > 0 && pass < kMaxPasses; pass++) {
+  for (int pass = 0; top > 0; pass++) {
     const int width = top < 12 ? top : 12;
     const int shift = top - width;
     top = shift;
@@ -727,6 +734,10 @@ __device__ Threshold radix_threshold(SelShared<kThreads>& sh, ForKeys for_keys, 
     prefix |= sh.pick[0] << shift;
     pmask |= dmask << shift;
     need -= sh.pick[1];
+    if constexpr (kCoarse) {
+      *taken = k - need + sh.pick[2];
+      if (*taken <= enough) break;   // uniform
+    }
     if (sh.pick[2] == need) break;   // the whole bin is taken (uniform)
   }
   return {prefix, pmask, need};
@@ -982,20 +993,24 @@ __global__ __launch_bounds__(kSweepThreads) void topk_sweep_kernel(const TopkArg
 }
 
 // One workgroup per row that looks at each key once.  A sample of 4096 keys
-// gives a bound T below the k-th largest key (the sample's rank k * 4096 /
-// len plus eight times its square root, so that 1.3 k to 2.5 k of the row's keys
-// lie at or above T); one pass over the row appends their positions to a list
-// in LDS; the radix select runs on the list alone; bitmaps of the row put the
-// selection in position order.  A pass over the row costs about 6 VALU
-// instructions per key, where the radix passes and the compaction of the
-// chunk stage cost 25, and nothing but the selection is written: 2048 rows x
-// 65536 positions read their 537 MB in 150 us (chunk and final stages 251).
-// When the bound's bin holds more than the list (heavy ties), the sample's exact
-// key of that rank takes its place, and if the keys above it are too few the
-// first positions equal to it complete them; a sample that still misleads
-// sends the row through sweep_row.  So ties cost a second pass (64 rows x 65536
-// of three distinct values 31 -> 29 us, 1 row 19 -> 28, one value everywhere 8
-// -> 22).
+// gives a bound T below the k-th largest key: the sample's key of rank k * 4096
+// / len plus eight times its square root plus 8, down to the lower edge of its
+// radix bin.  One pass over the row appends the positions of the keys at or
+// above T to a list in LDS, about rank * len / 4096 of them and the rest of the
+// bin (k = 512: 680 to 1000 of 4097 columns, 1360 of 65536, 1800 of 131072; k =
+// 32: 340 of 65536); the radix select runs on the list alone; bitmaps of the row
+// put the selection in position order.  A pass over the row costs about 6
+// VALU instructions per key, where the radix passes and the compaction of the
+// chunk stage cost 25, and nothing but the selection is written.
+// Where the sample puts more keys at the bound than the list holds, the bound
+// is the sample's exact key of that rank: the pass lists the keys above it and
+// marks the positions equal to it in a bitmap of the row, the first of which
+// complete a list of fewer than k, in the same pass.  A sample that misleads (too
+// few keys, or more than the list holds) sends the row through sweep_row.
+// Against the chunk and final stages, k = 512, rows x positions: 99 % of -inf 1 x
+// 16384 28.1 / 20.8 us and 64 x 65536 58.6 / 33.4; three values 13.8 / 13.4 and 29.9 /
+// 22.3; one value 7.1 / 8.2 and 10.6 / 18.5, which the stages see at once, each of
+// its chunk; ascending 9.5 / 11.2 and 15.4 / 17.7.
 constexpr int kListKeys = 4096;       // sample size and list capacity
 constexpr int kRowMaxLen = 131072;    // two bitmaps in the histograms' LDS
 constexpr int kRowMaxK = 1024;
@@ -1005,7 +1020,7 @@ __device__ __forceinline__ float key_value(uint32_t key) {   // inverse of order
 }
 
 template <int kThreads>
-__global__ __launch_bounds__(kThreads) void topk_row_kernel(
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kThreads == 1024 ? 8 : 1))) void topk_row_kernel(
     const float* p_logits, int64_t p_sl, const int32_t* p_lengths, int p_max_len, int p_k, int p_vec, int p_next_n,
     int32_t* p_out, int64_t p_so) {
   constexpr int P = kListKeys / kThreads;      // list keys per thread
@@ -1013,11 +1028,7 @@ __global__ __launch_bounds__(kThreads) void topk_row_kernel(
   constexpr int kVecs = 4;                     // 4-key loads per thread and step of the pass over the row
   __shared__ SelShared<kThreads> sh;
   __shared__ int32_t list[kListKeys];
-  // Counters.  `listed` is read by every thread after list_keys' last barrier
-  // and set to 0 again only behind another one (those of radix_threshold); the
-  // ties have a counter of their own, since no barrier lies between that read
-  // and their first count.
-  __shared__ uint32_t listed, tied;
+  __shared__ uint32_t listed;   // set to 0 once, before the first barrier
   const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
   const int len = clamp_len(p_lengths, p_max_len, row, p_next_n);
   const int k = p_k;
@@ -1047,6 +1058,8 @@ __global__ __launch_bounds__(kThreads) void topk_row_kernel(
 
   // The pass over the row: positions of the keys that `takes` picks go to the
   // list, and to `listed` their number (an unfinished one past the capacity).
+  // With kTies the positions equal to `tie` are set in the bitmap eq: a word of
+  // 32 positions is held by 8 consecutive lanes, whose last writes it whole.
   constexpr int kStep = kThreads * 4 * kVecs;
   auto load_step = [&](int base, float4 (&f)[kVecs]) {
 #pragma unroll
@@ -1075,13 +1088,31 @@ __global__ __launch_bounds__(kThreads) void topk_row_kernel(
     return hits;
   };
   auto hit_pos = [&](int base, int b) { return base + ((b >> 2) * kThreads + tid) * 4 + (b & 3); };
-  auto list_keys = [&](auto takes) {
+  uint32_t* gt = sh.hist[0];   // a bitmap of the keys above the threshold and one of those at it
+  uint32_t* eq = sh.hist[1];
+  const int words = (len + 31) / 32;
+  auto list_keys = [&](auto with_ties, auto takes, uint32_t tie) {
+    constexpr bool kTies = decltype(with_ties)::value;
     float4 cur[kVecs], nxt[kVecs];
     load_step(0, cur);
     bool room = true;   // uniform over the wave
     for (int base = 0; base < len && room; base += kStep) {
       if (base + kStep < len) load_step(base + kStep, nxt);
       uint32_t hits = hits_of(cur, takes);
+      if constexpr (kTies) {
+        const uint32_t at = hits_of(cur, [&](float v) { return order_key(v) == tie; });
+#pragma unroll
+        for (int q = 0; q < kVecs; q++) {
+          const int p = base + (q * kThreads + tid) * 4;
+          uint32_t m = (at >> (4 * q)) & 15u;
+          m <<= 4 * (lane & 7);
+          m |= dpp_or_zero<0xB1, 0xf>(m);    // lane ^ 1
+          m |= dpp_or_zero<0x4E, 0xf>(m);    // lane ^ 2
+          m |= dpp_or_zero<0x114, 0xf>(m);   // lane - 4
+          // a NaN's key also stands past the row's end
+          if ((lane & 7) == 7 && p < words * 32) eq[p >> 5] = (p | 31) < len ? m : m & ~(~0u << (len & 31));
+        }
+      }
       const uint32_t n = __popc(hits);
       const uint32_t incl = wave_incl_scan(n);
       const uint32_t total = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(incl), 63));
@@ -1105,11 +1136,24 @@ __global__ __launch_bounds__(kThreads) void topk_row_kernel(
     return static_cast<int>(listed);
   };
 
-  // ---- the bound T from a sample: runs of 4 keys at 1024 even places
+  // ---- the bound T from a sample: a run of 4 keys from each of 1024 equal
+  // parts of the row, at a place that differs from part to part: a row that
+  // repeats with the parts' length is not sampled at one phase (64 rows x 65536
+  // positions, the first 4 of every 64 low: 50 -> 15 us).  Neighbouring keys are
+  // often close, and lanes that count into one bin wait for each other, so at
+  // 1024 threads (few rows, a chain of phases) only eight lanes take neighbouring
+  // parts and a wave's eight eights lie apart (one ascending row of 16384: 12.5
+  // -> 11.2 us); at 512 (many rows) the spread loads cost more than the waits
+  // (1000 x 16384: 29.4 / 30.7).
   auto load_sample = [&](float (&f)[P]) {
+    constexpr uint32_t kParts = kListKeys / 4;
+    const uint32_t width = static_cast<uint32_t>(len) / kParts;   // at least 4
 #pragma unroll
     for (int q = 0; q < kRuns; q++) {
-      const float* s = x + ((static_cast<uint32_t>(q * kThreads + tid) * static_cast<uint32_t>(len) / (kListKeys / 4)) & ~3u);
+      const uint32_t n = q * kThreads + tid;
+      const uint32_t i = kThreads == 1024 ? ((n & 56) << 4) | (n >> 6 << 3) | (n & 7) : n;
+      const uint32_t at = ((i * 159u & 255u) * (width - 3)) >> 8;   // at most width - 4: the run stays in its part
+      const float* s = x + ((i * static_cast<uint32_t>(len) / kParts + at) & ~3u);
       if (p_vec) {
         const float4 v = *reinterpret_cast<const float4*>(s);
         f[4 * q] = v.x; f[4 * q + 1] = v.y; f[4 * q + 2] = v.z; f[4 * q + 3] = v.w;
@@ -1119,7 +1163,18 @@ __global__ __launch_bounds__(kThreads) void topk_row_kernel(
       }
     }
   };
-  auto sample_keys = [&](const float (&f)[P], uint32_t& kmin, uint32_t& kmax) {
+  const float share = static_cast<float>(kListKeys) / static_cast<float>(len);
+  const float mean = static_cast<float>(k) * share;
+  const uint32_t rank = static_cast<uint32_t>(min(static_cast<int>(mean + 8.f * __builtin_sqrtf(mean) + 8.f), kListKeys));
+  // sample keys that stand for three quarters of the list: three standard deviations short of it at kRowMaxLen
+  const uint32_t enough = max(rank, static_cast<uint32_t>(kListKeys / 4 * 3 * share));
+  uint32_t kmin, kmax, taken;
+  Threshold bound;
+  {
+    float f[P];
+    load_sample(f);
+    clear_hist(sh);
+    if (tid == 0) listed = 0;
     kmin = ~0u;
     kmax = 0u;
 #pragma unroll
@@ -1128,118 +1183,84 @@ __global__ __launch_bounds__(kThreads) void topk_row_kernel(
       kmin = min(kmin, kk[j]);
       kmax = max(kmax, kk[j]);
     }
-  };
-  const float mean = static_cast<float>(k) * kListKeys / static_cast<float>(len);
-  const uint32_t rank = static_cast<uint32_t>(min(static_cast<int>(mean + 8.f * __builtin_sqrtf(mean) + 8.f), kListKeys));
-  uint32_t kmin, kmax;
-  float bound;
-  {
-    float f[P];
-    load_sample(f);
-    clear_hist(sh);
-    if (tid == 0) listed = tied = 0;
-    sample_keys(f, kmin, kmax);
-    // one pass: the bin the rank falls in, whole
-    const Threshold t = radix_threshold<kThreads, 1>(sh, [&](auto f) { for_each_key(kk, f); }, rank, kmin, kmax);
-    bound = key_value(t.thr & t.pmask);
+    bound = radix_threshold<kThreads, true>(sh, [&](auto f) { for_each_key(kk, f); }, rank, kmin, kmax, enough, &taken);
   }
-  int n_list = list_keys([&](float v) { return v >= bound; });   // a NaN bound lists none
-  uint32_t ties = ~0u;   // the key whose first positions complete the list (none: the list holds the top k)
-  if (n_list > kListKeys) {   // uniform: many keys in the bin -- the sample's exact key of that rank, and the keys above it
-    float f[P];
-    load_sample(f);
-    clear_hist(sh);
-    sample_keys(f, kmin, kmax);
-    const Threshold t = radix_threshold(sh, [&](auto f) { for_each_key(kk, f); }, rank, kmin, kmax);
-    if (tid == 0) listed = 0;   // the first count was read before radix_threshold's barriers
-    __syncthreads();
-    n_list = list_keys([&](float v) { return order_key(v) > t.thr; });
-    if (n_list < k) ties = t.thr;
+  const bool ties = taken > enough;   // uniform: too many keys at the bound, which is exact then
+  int n_list;
+  if (ties) {
+    for (int i = tid; i < words; i += kThreads) gt[i] = 0u;   // the histograms' last reader is behind a barrier
+    n_list = list_keys(std::true_type{}, [&](float v) { return order_key(v) > bound.thr; }, bound.thr);
+  } else {
+    // a bin that reaches below the key of -inf, into the NaNs': every number
+    const float low = bound.thr < 0x007fffffu ? -__builtin_inff() : key_value(bound.thr);
+    n_list = list_keys(std::false_type{}, [&](float v) { return v >= low; }, 0u);
   }
-  uint32_t* gt = sh.hist[0];   // later: a bitmap of the keys above the threshold and one of those at it
-  uint32_t* eq = sh.hist[1];
-  const int words = (len + 31) / 32;
-  if (ties != ~0u) {
-    // The list holds every key above `ties`: the first k - n_list positions
-    // of that key complete it, collected step by step from the row's start.
-    for (int i = tid; i < words; i += kThreads) gt[i] = eq[i] = 0u;
-    __syncthreads();
-    for (int i = tid; i < n_list; i += kThreads) atomicOr(&gt[list[i] >> 5], 1u << (list[i] & 31));
-    int found = 0;
-    for (int base = 0; base < len && found < k - n_list; base += kStep) {
-      float4 cur[kVecs];
-      load_step(base, cur);
-      uint32_t hits = hits_of(cur, [&](float v) { return order_key(v) == ties; });
-      const uint32_t n = wave_incl_scan(__popc(hits));
-      if (lane == 63 && n) atomicAdd(&tied, n);
-      while (hits) {
-        const int b = __builtin_ctz(hits);
-        hits &= hits - 1;
-        const int p = hit_pos(base, b);
-        if (p < len) atomicOr(&eq[p >> 5], 1u << (p & 31));   // a NaN key (0) also stands past the row's end
+  if (n_list <= kListKeys && (ties || n_list >= k)) {   // uniform
+    uint32_t need = static_cast<uint32_t>(k - n_list);   // of the keys at the threshold
+    if (n_list < k) {
+      // the list holds every key above the bound, and eq the keys at it
+      for (int i = tid; i < n_list; i += kThreads) atomicOr(&gt[list[i] >> 5], 1u << (list[i] & 31));
+    } else {
+      // ---- the k largest of the list
+      int pos[P];
+#pragma unroll
+      for (int j = 0; j < P; j++) pos[j] = list[j * kThreads + tid < n_list ? j * kThreads + tid : 0];
+      float f[P];
+#pragma unroll
+      for (int j = 0; j < P; j++) f[j] = x[pos[j]];
+      clear_hist(sh);
+      kmin = ~0u;
+      kmax = 0u;
+#pragma unroll
+      for (int j = 0; j < P; j++) {
+        const bool ok = j * kThreads + tid < n_list;
+        kk[j] = ok ? order_key(f[j]) : 0u;
+        if (ok) { kmin = min(kmin, kk[j]); kmax = max(kmax, kk[j]); }
       }
+      const Threshold t =
+          radix_threshold(sh, [&](auto f) { for_each_key(kk, f); }, static_cast<uint32_t>(k), kmin, kmax);
+      need = t.need;
+      // the bitmaps take the histograms' place
+      for (int i = tid; i < words; i += kThreads) gt[i] = eq[i] = 0u;
       __syncthreads();
-      found = static_cast<int>(tied);
-      __syncthreads();   // before the next step's counts
+#pragma unroll
+      for (int j = 0; j < P; j++) {
+        const uint32_t m = kk[j] & t.pmask;
+        if (kk[j] != 0u && m >= t.thr) atomicOr(m > t.thr ? &gt[pos[j] >> 5] : &eq[pos[j] >> 5], 1u << (pos[j] & 31));
+      }
     }
-    if (found < k - n_list) ties = ~0u;   // uniform
-  }
-  if (ties == ~0u && (n_list < k || n_list > kListKeys)) {   // uniform: the sample misled
     __syncthreads();
-    sweep_row<kThreads, P>(sh, x, len, k, p_vec, out);
-    return;
-  }
-  uint32_t need = static_cast<uint32_t>(k - n_list);   // of the keys at the threshold
-  if (ties == ~0u) {
-    // ---- the k largest of the list
-    int pos[P];
-#pragma unroll
-    for (int j = 0; j < P; j++) pos[j] = list[j * kThreads + tid < n_list ? j * kThreads + tid : 0];
-    float f[P];
-#pragma unroll
-    for (int j = 0; j < P; j++) f[j] = x[pos[j]];
-    clear_hist(sh);
-    kmin = ~0u;
-    kmax = 0u;
-#pragma unroll
-    for (int j = 0; j < P; j++) {
-      const bool ok = j * kThreads + tid < n_list;
-      kk[j] = ok ? order_key(f[j]) : 0u;
-      if (ok) { kmin = min(kmin, kk[j]); kmax = max(kmax, kk[j]); }
-    }
-    const Threshold t = radix_threshold(sh, [&](auto f) { for_each_key(kk, f); }, static_cast<uint32_t>(k), kmin, kmax);
-
-    need = t.need;
-    // the bitmaps take the histograms' place (their last reader is behind a barrier)
-    for (int i = tid; i < words; i += kThreads) gt[i] = eq[i] = 0u;
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < P; j++) {
-      const uint32_t m = kk[j] & t.pmask;
-      if (kk[j] != 0u && m >= t.thr) atomicOr(m > t.thr ? &gt[pos[j] >> 5] : &eq[pos[j] >> 5], 1u << (pos[j] & 31));
+    // ---- the selection in position order
+    constexpr int kEqBits = 18;   // up to kRowMaxLen keys at the threshold, and kListKeys above it
+    static_assert(kRowMaxLen < 1 << kEqBits && kListKeys < 1 << (32 - kEqBits));
+    constexpr uint32_t kEqMask = (1u << kEqBits) - 1;
+    const int per = (words + kThreads - 1) / kThreads;   // consecutive words of this thread
+    const int w0 = min(tid * per, words), w1 = min(w0 + per, words);
+    uint32_t n = 0;
+    for (int i = w0; i < w1; i++)
+      n += (static_cast<uint32_t>(__popc(gt[i])) << kEqBits) | static_cast<uint32_t>(__popc(eq[i]));
+    uint32_t all;
+    const uint32_t before = block_excl_scan(sh, n, &all);
+    if ((all & kEqMask) >= need) {   // uniform: false where the keys at the bound and above are fewer than k
+      uint32_t r = before & kEqMask;                     // keys at the threshold seen so far
+      uint32_t o = (before >> kEqBits) + min(r, need);
+      for (int i = w0; i < w1; i++) {
+        const uint32_t g = gt[i], e = eq[i];
+        uint32_t bits = r < need ? g | e : g;
+        while (bits) {
+          const int b = __builtin_ctz(bits);
+          bits &= bits - 1;
+          const bool at = (e >> b) & 1;
+          if (!at || r < need) out[o++] = 32 * i + b;
+          r += at;
+        }
+      }
+      return;
     }
   }
+  // the sample misled
   __syncthreads();
-  // ---- the selection in position order
-  const int per = (words + kThreads - 1) / kThreads;   // consecutive words of this thread
-  const int w0 = min(tid * per, words), w1 = min(w0 + per, words);
-  uint32_t n = 0;
-  for (int i = w0; i < w1; i++) n += (static_cast<uint32_t>(__popc(gt[i])) << 16) | static_cast<uint32_t>(__popc(eq[i]));
-  uint32_t all;
-  const uint32_t before = block_excl_scan(sh, n, &all);
-  uint32_t r = before & 0xffffu;                       // keys at the threshold seen so far
-  uint32_t o = (before >> 16) + min(r, need);
-  for (int i = w0; i < w1; i++) {
-    const uint32_t g = gt[i], e = eq[i];
-    uint32_t bits = g | e;
-    while (bits) {
-      const int b = __builtin_ctz(bits);
-      bits &= bits - 1;
-      const bool at = (e >> b) & 1;
-      if (!at || r < need) out[o++] = 32 * i + b;
-      r += at;
-    }
-  }
+  sweep_row<kThreads, P>(sh, x, len, k, p_vec, out);
 }
 
 bool aligned(const void* p, uintptr_t n) { return (reinterpret_cast<uintptr_t>(p) & (n - 1)) == 0; }

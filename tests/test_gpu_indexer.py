@@ -563,3 +563,25 @@ def test_next_n_rows_share_loads(cuda, next_n, H):
             pools = indexer_decode_pool_topk(q, cache, w, ctx, bt, max_len, k=k)
             cap = min(max_len, per_req * bs)
             assert torch.equal(pools, indexer_topk(want[:, :cap], rows_ctx, min(k, cap)))
+
+
+@pytest.mark.parametrize("rows,n", [(64, 131072), (22, 65537), (16, 57344), (15, 65537), (256, 4097)])
+def test_topk_one_value_rows(cuda, rows, n):
+    """Rows that are one value but for a few keys above it, at the longest row
+    of the one-workgroup selection (every position of 131072 tied), at the row
+    counts where long rows change plan, and short rows: the keys above and the
+    first positions of the tie."""
+    import torch
+    from sparse_indexer import indexer_topk
+    x = torch.full((rows, n), -0.25, device=cuda)
+    x[1, 5::n // 100] = 1.0
+    x[2, n - 300:] = float("inf")
+    x[3] = -float("inf")
+    x[4] = float("nan")
+    x[4, n - 200:] = -float("inf")
+    log_case("indexer top-k one value", rows, n)
+    got = indexer_topk(x, torch.full((rows,), n, dtype=torch.int32, device=cuda), 512).cpu().numpy()
+    for r in range(rows):
+        above = {1: np.arange(5, n, n // 100), 2: np.arange(n - 300, n), 4: np.arange(n - 200, n)}.get(r, np.arange(0))
+        ties = np.setdiff1d(np.arange(1024), above)[:512 - len(above)]
+        assert np.array_equal(got[r], np.sort(np.concatenate([above, ties]))), r

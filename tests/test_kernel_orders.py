@@ -74,3 +74,36 @@ def test_topk_any_order_other_plans(lib, oracle, order):
         x = rows_of(n, k)[1:4]
         lens = np.array([n, n - 5, n], np.int32)
         assert np.array_equal(topk(lib, x, lens, k, n), oracle.indexer_topk(x, lens, k)), (n, k)
+
+
+def sampled(n):
+    """The 4096 positions of a row of n columns that the one-workgroup
+    selection ranks for its bound (either workgroup size takes the same)."""
+    part = np.arange(1024)
+    at = (part * n // 1024 + ((part * 159 & 255) * (n // 1024 - 3) >> 8)) & ~3
+    return (at[:, None] + np.arange(4)).reshape(-1)
+
+
+# n, k, rows of the call: 1024 threads, 512 threads, and a length with more parts than columns to a run
+@pytest.mark.parametrize("n,k,rows", [(16384, 512, 6), (9001, 1024, 256), (40000, 1024, 24)])
+def test_topk_misleading_sample(lib, oracle, n, k, rows):
+    """Rows whose sample says the wrong thing: the sampled keys below all
+    others (the list overflows) or above them (too few listed), one sampled
+    value whose copies complete the list, too few copies of it, NaN all over
+    the sample, and a row that repeats with the parts' length."""
+    lib.host_hip_order(0, 0)
+    rng = np.random.default_rng(n)
+    x = np.zeros((rows, n), np.float32)
+    x[:6] = rng.standard_normal((6, n))
+    s = sampled(n)
+    assert len(np.unique(s)) == 4096 and s.max() < n
+    x[0, s] -= 20
+    x[1, s] += np.where(np.arange(4096) < k // 2, 20, 0)
+    x[2, s] = 5
+    x[3, s[::8][:k - 300]] = 5
+    x[4, s] = np.nan
+    x[5, np.arange(n) % (n // 1024) < 4] -= 6
+    lens = np.zeros(rows, np.int32)
+    lens[:6] = n
+    got = topk(lib, x, lens, k, n)
+    assert np.array_equal(got[:6], oracle.indexer_topk(x[:6], lens[:6], k))
