@@ -1482,17 +1482,22 @@ TopkPlan plan_topk(int64_t num_rows, int64_t max_len, int64_t k) {
 
 // Rows that topk_row_kernel takes whatever plan_topk says of them (its
 // workspace is asked for all the same and stays unused).  Against the chunk
-// and final stages, k = 512: 2048 rows x 65536 positions 251 -> 150 us, x
-// 16384 87 -> 50, 500 x 16000 27 -> 16.3, 48 x 12000 17.8 -> 10.2, 16 x 65536
-// 19.4 -> 13.9, 1 x 16384 12.2 -> 10.0.  A few long rows keep the two stages: one
-// compute unit streams a row that other XCDs have just written more slowly than
-// several do (a one-token decode layer over 65536 pools 40.1 -> 42.3 us with
-// this kernel, 8 tokens over 32768 79.4 -> 79.7), whatever a repeated call alone
-// says (14.0 -> 12.5).  512 threads leave three rows to a CU where many short
-// rows queue (2048 x 8192: 35 us against 48 with 1024 threads, x 16384 50 / 53, x
-// 32768 98 / 95; below 256 rows each has a CU to itself and 1024 threads are ahead).
+// and final stages, k = 512, us: 2048 rows x 65536 positions 230 / 154, x 16384 79 /
+// 53, 600 x 12000 42 / 18, 48 x 12000 17.3 / 10.0, 24 x 65536 14.8 / 13.8, 1 x 16384
+// 11.6 / 9.7.  A few long rows keep the two stages, which put several compute
+// units on a row: the kernel reads 0.5 MB per row through one (16 x 131072 16.9 /
+// 19.4, with k = 32 13.3 / 16.8; 24 x 131072 and k = 1 13.4 / 17.3, 48 17.0 / 17.8, 64 20.8 /
+// 18.1; 16 x 65536 and k = 1 10.3 / 11.3, 20 and more ahead at every k; 16 x 50000 ahead):
+// from 16 rows up to 57344 positions, then one row more per 1536.  Below 16 rows
+// one unit streams a row that other XCDs have just written more slowly than
+// several do (a one-token decode layer over 65536 pools 40.1 / 42.3 us, 8
+// tokens over 32768 79.4 / 79.7), whatever a repeated call alone says (14.0 /
+// 12.5).  512 threads leave three rows to a CU where many short rows queue (2048 x
+// 8192: 35 us against 48 with 1024 threads, x 16384 50 / 53, x 32768 98 / 95; below
+// 256 rows each has a CU to itself and 1024 threads are ahead).
 bool row_plan(int64_t num_rows, int64_t max_len, int64_t k) {
-  return max_len > kListKeys && max_len <= kRowMaxLen && k <= kRowMaxK && (max_len <= 16384 || num_rows >= 16);
+  if (max_len <= kListKeys || max_len > kRowMaxLen || k > kRowMaxK) return false;
+  return max_len <= 16384 || (num_rows >= 16 && 1536 * num_rows >= max_len - 32768);
 }
 
 int64_t topk_ws_bytes(const TopkPlan& p, int64_t rows, int64_t k) {
