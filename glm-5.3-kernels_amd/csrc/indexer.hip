@@ -519,7 +519,13 @@ void fp8_mqa_logits_rows_kernel(const LogitsArgs a, int num_tokens) {
       __builtin_amdgcn_sched_barrier(0);
     }
   }
-  if (chunks > 0) store_chunk(chunks - 1);
+  if (chunks > 0) {
+    // the last chunk's results are other lanes' writes, with no workgroup barrier since
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    store_chunk(chunks - 1);
+  }
   if (a.clean) {   // the run past every row's context
 #pragma unroll
     for (int r = 0; r < kR; r++)

@@ -107,3 +107,33 @@ def test_topk_misleading_sample(lib, oracle, n, k, rows):
     lens[:6] = n
     got = topk(lib, x, lens, k, n)
     assert np.array_equal(got[:6], oracle.indexer_topk(x[:6], lens[:6], k))
+
+
+@pytest.mark.parametrize("order", ORDERS)
+@pytest.mark.parametrize("heads,tokens,keys,clean", [(16, 17, 130, 1), (32, 16, 200, 0)])
+def test_logits_rows_any_order(lib, heads, tokens, keys, clean, order):
+    """The logits of rows that share one block table (keys staged in LDS,
+    results handed between lanes for the stores) against the same rows with a
+    table each: bit-identical, whichever lane of a wave runs first."""
+    fn = lib.glm53_fp8_paged_mqa_logits
+    fn.argtypes = [P, I64, I64, P, I64, I64, I64, P, I64, P, P, I64, I64, I64, I64, I64, I64, ctypes.c_int, P, I64, P]
+    lib.host_hip_order(*order)
+    rng = np.random.default_rng(heads + keys)
+    block, pages = 16, (keys + 15) // 16
+    q = rng.integers(0, 120, tokens * heads * 128 + 16, dtype=np.uint8)     # E4M3 of either sign, no NaN
+    q ^= (rng.random(q.shape) < 0.5).astype(np.uint8) << 7
+    kv = rng.integers(0, 120, pages * block * 132 + 16, dtype=np.uint8)
+    qa, kva = (a.ctypes.data + 15 & ~15 for a in (q, kv))
+    page = kv[kva - kv.ctypes.data:][:pages * block * 132].reshape(pages, block * 132)
+    page[:, block * 128:] = (rng.random((pages, block), dtype=np.float32) - 0.2).view(np.uint8)
+    w = rng.standard_normal((tokens, heads)).astype(np.float32)
+    lens = rng.integers(0, keys + 1, tokens).astype(np.int32)
+    lens[0] = keys
+    table = rng.permutation(pages).astype(np.int32)
+    out = []
+    for bt, stride in ((table, 0), (np.tile(table, (tokens, 1)), pages)):
+        o = np.full((tokens, keys), 7, np.float32)
+        assert fn(qa, heads * 128, 128, kva, block * 132, block, pages, w.ctypes.data, heads, lens.ctypes.data,
+                  bt.ctypes.data, stride, pages, tokens, heads, 128, keys, clean, o.ctypes.data, keys, None) == 0
+        out.append(o)
+    assert np.array_equal(out[0], out[1])
