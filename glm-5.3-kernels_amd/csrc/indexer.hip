@@ -36,12 +36,15 @@
 // digits (LDS histograms) for the k-th largest key, then an ordered
 // compaction (two workgroup scans) that writes the selected positions in
 // ascending order, ties at the threshold resolved by position:
-// deterministic.  One workgroup per row is bound by its CU's vector rate, so
-// long rows run in two stages: workgroups (row, chunk) keep each chunk's
-// local top-k in position order (a key of the row's top k is in its chunk's
-// top k), then one workgroup per row selects from those candidates.  Keys
-// stay in registers (thread-contiguous runs of positions) through every
-// pass; rows too long for the two stages are re-read from L2 per pass.
+// deterministic.  Rows of at most 4096 positions are selected by one workgroup
+// with the row in registers.  Many or shorter rows up to 131072 positions
+// (row_plan): one workgroup per row that passes over it once with a sampled
+// bound (topk_row_kernel).  Few long rows, longer rows and k > 1024 run in two
+// stages: workgroups (row, chunk) keep each chunk's local top-k in position
+// order (a key of the row's top k is in its chunk's top k), then one workgroup
+// per row selects from those candidates.  Keys stay in registers (thread-contiguous
+// runs of positions) through every pass; rows too long for the two stages
+// are re-read from L2 per pass.
 #include <type_traits>
 
 #include "glm53_common.h"
@@ -68,8 +71,8 @@ struct LogitsArgs {
   int num_blocks;
   const float* w;           // [T][H]
   int64_t sw_t;
-  const int32_t* ctx;       // [T] pool-granular context lengths
-  const int32_t* bt;        // [T][max_blocks]
+  const int32_t* ctx;       // [T / next_n] pool-granular context lengths of each request's last row
+  const int32_t* bt;        // [T / next_n][max_blocks]
   int64_t bt_stride;
   int max_blocks;
   int num_heads;
@@ -334,8 +337,8 @@ __global__ __launch_bounds__(kLogitThreads) void fp8_paged_mqa_logits_kernel(
 // product holds the VALU for a third less time), issued two steps ahead of
 // their clamps with no wait between, operands read from LDS a group ahead,
 // masks and stores once per chunk (16 bytes per lane).  2048 rows x 65536
-// pools, 32 heads: 650 -> 465 us (2.35 PFLOP/s of FP8); with the top-512
-// 863 -> 706 us, 500 rows x 16000 pools 80.0 -> 65.6 us.
+// pools, 32 heads: 650 -> 465 to 533 us by the card (2.06 to 2.35 PFLOP/s of FP8);
+// 500 rows x 16000 pools 42 us.
 constexpr int kRowsRun = 1024;         // keys of a workgroup: 64 groups, one per lane of the table lookup
 constexpr int kRowsChunk = 4;          // 16-key groups per chunk, one staged by each wave
 constexpr int kRowsBufs = 2;
@@ -445,7 +448,8 @@ void fp8_mqa_logits_rows_kernel(const LogitsArgs a, int num_tokens) {
   // anywhere in the run when cleaning).
   const int limit = t0 + g < num_tokens ? (a.clean ? j_end : min(j_end, my_len)) : 0;
   float* const out = a.logits + static_cast<int64_t>(min(t0 + g, num_tokens - 1)) * a.sl_t + j_run + 4 * c;
-  const bool vec = (reinterpret_cast<uintptr_t>(a.logits) & 15) == 0 && (a.sl_t & 3) == 0;   // runs start at multiples of 64
+  // runs start at multiples of 64
+  const bool vec = (reinterpret_cast<uintptr_t>(a.logits) & 15) == 0 && (a.sl_t & 3) == 0;
   auto store_chunk = [&](int ch) {
     const int j = j_run + 64 * ch + 4 * c;
     float4 v = *reinterpret_cast<const float4*>(&sh.res[w][g][4 * c]);
@@ -1026,7 +1030,8 @@ __device__ __forceinline__ float key_value(uint32_t key) {   // inverse of order
 }
 
 template <int kThreads>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kThreads == 1024 ? 8 : 1))) void topk_row_kernel(
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kThreads == 1024 ? 8 : 1)))
+void topk_row_kernel(
     const float* p_logits, int64_t p_sl, const int32_t* p_lengths, int p_max_len, int p_k, int p_vec, int p_next_n,
     int32_t* p_out, int64_t p_so) {
   constexpr int P = kListKeys / kThreads;      // list keys per thread
@@ -1171,7 +1176,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kThrea
   };
   const float share = static_cast<float>(kListKeys) / static_cast<float>(len);
   const float mean = static_cast<float>(k) * share;
-  const uint32_t rank = static_cast<uint32_t>(min(static_cast<int>(mean + 8.f * __builtin_sqrtf(mean) + 8.f), kListKeys));
+  const int above = static_cast<int>(mean + 8.f * __builtin_sqrtf(mean) + 8.f);
+  const uint32_t rank = static_cast<uint32_t>(min(above, kListKeys));
   // sample keys that stand for three quarters of the list: three standard deviations short of it at kRowMaxLen
   const uint32_t enough = max(rank, static_cast<uint32_t>(kListKeys / 4 * 3 * share));
   uint32_t kmin, kmax, taken;
@@ -1371,7 +1377,8 @@ extern "C" int glm53_fp8_paged_mqa_logits_next_n(const void* q, int64_t sq_t, in
   if (!q || !kv_cache || !weights || !context_lens || !block_table || !logits) return GLM53_ERR_NULL_POINTER;
   if (next_n < 1 || next_n > 65535 || num_requests < 0 || num_requests > 65535) return GLM53_ERR_BAD_SHAPE;
   const int64_t num_tokens = num_requests * next_n;
-  if (head_dim != kHeadDim || num_heads < 16 || num_heads > kMaxHeads || num_heads % 16 || num_tokens > 65535 || block_size < 1 || num_blocks < 1 || num_blocks > (int64_t(1) << 31) - 1 ||
+  if (head_dim != kHeadDim || num_heads < 16 || num_heads > kMaxHeads || num_heads % 16 || num_tokens > 65535 ||
+      block_size < 1 || num_blocks < 1 || num_blocks > (int64_t(1) << 31) - 1 ||
       max_blocks < 1 || max_len < 0 || max_len > (int64_t(1) << 30) ||
       max_blocks * block_size > (int64_t(1) << 31) - 1 || page_bytes < block_size * (kHeadDim + 4) ||
       sq_h < kHeadDim || sq_t < num_heads * sq_h || sw_t < num_heads || sl_t < max_len ||
@@ -1394,7 +1401,8 @@ extern "C" int glm53_fp8_paged_mqa_logits_next_n(const void* q, int64_t sq_t, in
                  static_cast<int>(max_len), 0, logits, sl_t, clean_logits ? 1 : 0, 1, 1};
     const int64_t row_blocks = (num_tokens + 4 * kLogitWaves - 1) / (4 * kLogitWaves);
     a.keys_per_wg = rows_run(row_blocks, max_len);
-    const dim3 grid(static_cast<unsigned>((max_len + a.keys_per_wg - 1) / a.keys_per_wg), static_cast<unsigned>(row_blocks));
+    const dim3 grid(static_cast<unsigned>((max_len + a.keys_per_wg - 1) / a.keys_per_wg),
+                    static_cast<unsigned>(row_blocks));
     void (*kernel)(LogitsArgs, int);
     switch (num_heads / 16) {
       case 1: kernel = fp8_mqa_logits_rows_kernel<1>; break;
@@ -1441,9 +1449,10 @@ namespace {
 // candidates): B=8 16.4 -> 15.6 us, B=1 11.75 -> 11.66 us.  From 32 rows on
 // (throughput: the chunk stage alone is many workgroups per CU) 512-thread
 // workgroups over 8192-position chunks, half the workgroups and candidates
-// of 4096 (2048 rows x 65536 positions, k = 512: 283 -> 242 us; 32 rows
-// 16.6 -> 15.6 us; 16 rows 15.0 -> 15.5 us, so the latency choice stays
-// below 32).
+// of 4096 (k = 512, 65536 positions, measured before topk_row_kernel took
+// such rows: 2048 rows 283 -> 242 us, 32 rows 16.6 -> 15.6 us, 16 rows 15.0 -> 15.5
+// us, so the latency choice stays below 32).  That leaves it k > 1024, more
+// than 131072 positions, and 32 to 63 rows of 81921 positions and more.
 struct TopkPlan {
   enum Mode { kDirect, kChunked, kSweepMode } mode;
   int chunk_p, final_p, chunks, chunk_len, chunk_threads;
@@ -1550,7 +1559,9 @@ extern "C" int glm53_indexer_topk_next_n(const float* logits, int64_t sl, const 
                                          int64_t next_n, int64_t max_len, int64_t k, void* workspace,
                                          int64_t workspace_bytes, int32_t* out, int64_t so, void* stream) {
   if (!logits || !lengths || !out) return GLM53_ERR_NULL_POINTER;
-  if (next_n < 1 || next_n > (int64_t(1) << 30) || num_rows % next_n || !topk_shape_ok(num_rows, max_len, k) || sl < max_len || so < k) return GLM53_ERR_BAD_SHAPE;
+  if (next_n < 1 || next_n > (int64_t(1) << 30) || num_rows % next_n || !topk_shape_ok(num_rows, max_len, k) ||
+      sl < max_len || so < k)
+    return GLM53_ERR_BAD_SHAPE;
   if (num_rows == 0) return 0;
   if (!aligned(logits, 4)) return GLM53_ERR_MISALIGNED;
   const TopkPlan plan = plan_topk(num_rows, max_len, k);

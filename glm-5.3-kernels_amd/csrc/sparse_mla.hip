@@ -1002,9 +1002,10 @@ void sparse_mla_pair_kernel(const MlaArgs a) {
 // instructions per wave and unit set the time, with two barriers; from about
 // 1000 tokens on the row gathers do (T=1024: 164 us from L2-resident rows, 204
 // over a 262144-row cache, 5.8 TB/s of row bytes).  Against the pair kernel
-// below (262144-row cache, 2176 indices, us): 128 tokens 78 -> 40 (2 splits,
-// with the merge of few splits), 256 105 -> 57, 300 142 -> 89, 512 145 -> 107, 1100
-// 289 -> 248, 2048 418 -> 388; 48 tokens in 5 splits 36.2 -> 22.4.
+// above (one flat cache of 262144 rows, 2176 indices, us): 128 tokens 78 -> 40 (2
+// splits, with the merge of few splits), 256 105 -> 57, 300 142 -> 89, 512 145 ->
+// 107, 1100 289 -> 248, 2048 418 -> 388 (through the pools, 262144 rows: 371 -> 369);
+// 48 tokens in 5 splits 36.2 -> 22.4.  rows_waves has the choice.
 // 128-key units of 8 waves against 64-key units of 4, one split: 256 tokens 57
 // / 66, 300 100 / 89, 512 110 / 107, 640 154 / 158, 1024 214 / 204 -- by the rounds
 // they take on the compute units (one workgroup of 8 waves each, or two of 4).

@@ -76,7 +76,7 @@ def fp8_paged_mqa_logits(q: torch.Tensor, kv_cache: torch.Tensor, weights: torch
                                                  ctx.data_ptr(), bt.data_ptr(), bt_stride, bt.shape[1], B, next_n,
                                                  H, HEAD_DIM, max_model_len, int(bool(clean_logits)),
                                                  logits.data_ptr(), logits.stride(0), _lib.stream_handle(q.device))
-    _lib.check(rc, "glm53_fp8_paged_mqa_logits")
+    _lib.check(rc, "glm53_fp8_paged_mqa_logits_next_n")
     return logits
 
 
@@ -107,7 +107,7 @@ def _topk_rows(logits: torch.Tensor, lengths: torch.Tensor, next_n: int, k: int)
         rc = L.glm53_indexer_topk_next_n(logits.data_ptr(), logits.stride(0), lengths.contiguous().data_ptr(), rows,
                                          next_n, n, k, ws.data_ptr(), ws_bytes, out.data_ptr(), out.stride(0),
                                          _lib.stream_handle(logits.device))
-    _lib.check(rc, "glm53_indexer_topk")
+    _lib.check(rc, "glm53_indexer_topk_next_n")
     return out
 
 

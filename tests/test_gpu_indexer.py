@@ -488,12 +488,13 @@ def test_shared_table_run_edges(cuda, heads, bs, pools, T):
 
 
 @pytest.mark.parametrize("rows,n,k", [(9, 4097, 512), (9, 5001, 1024), (270, 8192, 512), (9, 12001, 1), (9, 65536, 1024),
-                                      (17, 131072, 512), (9, 131073, 512), (9, 20000, 1025)])
+                                      (17, 131072, 512), (9, 131073, 512), (9, 20000, 1025), (64, 131072, 512),
+                                      (24, 65536, 1024)])
 def test_topk_filtered_rows(cuda, oracle, rows, n, k):
     """The one-workgroup selection that filters a row by a sampled bound, at
-    the edges of its range (4097 and 131072 positions, k = 1024, unaligned
-    rows, rows shorter than its list or than k, 512 and 1024 threads) and the
-    plans just past them, on rows whose sample says little: few distinct
+    the edges of its range (4097 and, of 64 rows, 131072 positions, k = 1024,
+    unaligned rows, rows shorter than its list or than k, 512 and 1024 threads)
+    and the plans just past them (also few rows of 65536 and 131072), on rows whose sample says little: few distinct
     values, one value, NaN or -inf almost everywhere, ascending, a block of
     large keys, both zeros."""
     import torch

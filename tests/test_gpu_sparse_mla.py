@@ -580,8 +580,8 @@ def test_three_key_group_splits(cuda, oracle, small_cache):
 def test_long_split_pair_kernel_edges(cuda, oracle, small_cache):
     """Splits longer than one chunk (256 indices) in small batches (one
     online-softmax stream per split; a handful of workgroups takes the rows
-    kernel, test_long_split_by_workgroups has the pair kernel's range): against the reference's single stream
-    (groups=1, BLOCK_N=32) with odd tile counts (352 = 11 tiles, 288 = 9), a
+    kernel, test_long_split_by_workgroups has the pair kernel's range): against
+    the reference's single stream (groups=1, BLOCK_N=32) with odd tile counts (352 = 11 tiles, 288 = 9), a
     last split shorter than the others (1088 in 3 splits), split partials
     merged (2176 in 2 splits, 20 heads: a padded head group), pads and
     indices outside the cache both ways; all -1 gives exactly 0; an empty
@@ -596,11 +596,11 @@ def test_long_split_pair_kernel_edges(cuda, oracle, small_cache):
         q = torch.randn(T, H, 512, generator=g, device=cuda).to(torch.bfloat16)
         idx = torch.randint(-40, n + 40, (T, 1, topk), generator=g, device=cuda, dtype=torch.int32)
         idx[0, :, topk // 2:] = -1
-        log_case("mla pair kernel", T, H, topk, splits)
+        log_case("mla long splits, few workgroups", T, H, topk, splits)
         out = triton_mla_sparse_attention(q, kv, idx, W.SM_SCALE, num_kv_splits=splits)
         torch.cuda.synchronize()
         want = oracle.sparse_mla(u16(q), rows, idx.cpu().numpy(), W.SM_SCALE, n_splits=splits, groups=1, block_n=32)
-        compare(out, want, ("pair kernel", T, H, topk, splits))
+        compare(out, want, ("few workgroups", T, H, topk, splits))
         blank = triton_mla_sparse_attention(q, kv, torch.full_like(idx, -1), W.SM_SCALE, num_kv_splits=splits)
         assert torch.equal(blank, torch.zeros_like(blank)), (T, H, topk, splits)
     q = torch.randn(2, 16, 512, generator=g, device=cuda).to(torch.bfloat16)
@@ -620,8 +620,8 @@ def test_long_split_rows_kernel_edges(cuda, oracle, small_cache, T, H, topk, spl
     whole, half or a few keys, the first half of a row's indices masked (whole
     masked units before and after the first valid one), indices outside the
     cache both ways, 1 to 5 head groups with a padded one, 1 to 8 splits
-    through either merge, and the grids on both sides of each step of the
-    kernel choice; the paged form is bit-identical."""
+    through either merge; 600 and 800 workgroups of several splits and head
+    groups take the pair kernel; the paged form is bit-identical."""
     from titan_mla import triton_mla_sparse_attention, triton_mla_sparse_attention_paged
     w, rows = small_cache
     n = w["n_rows"]
