@@ -398,7 +398,8 @@ int glm53_fp8_paged_mqa_logits_next_n(const void* q, int64_t sq_t, int64_t sq_h,
  *   workspace  device scratch of glm53_indexer_topk_workspace_bytes(...) bytes
  *              (0 for rows of at most 4096 columns; may then be NULL); the
  *              size asked for num_rows rows serves every call with at most
- *              that many rows (same max_len and k)
+ *              that many rows (same max_len and k); calls that take one
+ *              workgroup per row require it too and leave it unused
  *   out        int32 [num_rows][k], row stride so
  */
 int64_t glm53_indexer_topk_workspace_bytes(int64_t num_rows, int64_t max_len,

@@ -84,7 +84,7 @@ def sampled(n):
     return (at[:, None] + np.arange(4)).reshape(-1)
 
 
-# n, k, rows of the call: 1024 threads, 512 threads, and a length with more parts than columns to a run
+# columns, k and rows of the call: 1024 threads, 512 threads, and few long rows
 @pytest.mark.parametrize("n,k,rows", [(16384, 512, 6), (9001, 1024, 256), (40000, 1024, 24)])
 def test_topk_misleading_sample(lib, oracle, n, k, rows):
     """Rows whose sample says the wrong thing: the sampled keys below all
